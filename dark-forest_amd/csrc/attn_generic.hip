@@ -1,12 +1,13 @@
-// attn_generic.hip — fp32 attention kernels for any d_head in 1..=128.
+// attn_generic.hip — fp32 attention backward without any scratch memory.
 //
-// The MFMA kernels cover d_head = 64 (GPT-2's head size and every config this
-// library is measured on). These kernels keep the reference's full argument
-// range (AttentionContext accepts 1 <= d_head <= 128, darkforest-cuda/src/lib.rs:1981)
-// and are exact fp32: one wave per (query row, head); lanes take 64 keys at a
-// time for the scores and the d columns for the accumulations. Unlike the
-// reference kernels (attention_fused.cu:111-112, 417-420) they are correct for
-// 64 < d_head <= 128 as well.
+// The reference's backward launchers take the caller's probability buffer,
+// which holds the row statistics that the fp32 kernels (attn_fp32.hip) need. A
+// NULL buffer, or a single-head one of one row (one float), is also accepted:
+// these calls take the kernel below, any d_head in 1..=128 in exact fp32, one
+// wave per (query row, head); lanes take 64 keys at a time for the scores and
+// the d columns for the accumulations. Unlike the reference kernels
+// (attention_fused.cu:111-112, 417-420) it is correct for 64 < d_head <= 128
+// as well.
 #include "dfattn_internal.h"
 
 namespace dfattn {
@@ -54,28 +55,6 @@ __device__ void row_forward(const float *qrow_lds, const float *__restrict__ K,
     }
     m = m_new;
   }
-}
-
-__global__ __launch_bounds__(256) void fwd_generic_kernel(
-    const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
-    float *__restrict__ O, float *__restrict__ LSE, int H, int S, int D, float scale,
-    int causal) {
-  __shared__ float qs[4][kMaxD];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * 4 + wave, head = blockIdx.y;
-  const size_t ld = (size_t)H * D, hoff = (size_t)head * D;
-  for (int d = lane; d < D; d += 64) qs[wave][d] = row < S ? Q[(size_t)row * ld + hoff + d] : 0.f;
-  __syncthreads();
-  if (row >= S) return;
-  const int kmax = causal ? row + 1 : S;
-  float m, l, o0, o1;
-  row_forward(qs[wave], K, V, ld, hoff, D, kmax, scale, lane, m, l, o0, o1);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  float *orow = O + (size_t)row * ld + hoff;
-  if (lane < D) orow[lane] = o0 * inv;
-  if (lane + 64 < D) orow[lane + 64] = o1 * inv;
-  if (LSE != nullptr && lane == 0)
-    LSE[(size_t)head * S + row] = l > 0.f ? m + logf(l) : -INFINITY;
 }
 
 // Backward of one row: recompute (m, l, o) to get lse and Delta = dO . O,
@@ -153,15 +132,6 @@ hipError_t fill_zero(float *p, size_t n, hipStream_t stream) {
 }
 
 }  // namespace
-
-hipError_t launch_fwd_generic(const float *q, const float *k, const float *v, float *o,
-                              float *lse, int n_heads, int seq_len, int d_head, float scale,
-                              bool causal, hipStream_t stream) {
-  const dim3 grid((seq_len + 3) / 4, n_heads);
-  hipLaunchKernelGGL(fwd_generic_kernel, grid, dim3(256), 0, stream, q, k, v, o, lse, n_heads,
-                     seq_len, d_head, scale, causal ? 1 : 0);
-  return hipGetLastError();
-}
 
 hipError_t launch_bwd_generic(const float *q, const float *k, const float *v, const float *d_o,
                               float *d_q, float *d_k, float *d_v, int n_heads, int seq_len,

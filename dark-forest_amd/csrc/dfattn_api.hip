@@ -3,7 +3,8 @@
 //
 // Kernel selection: d_head == 64 with 16-byte aligned tensors takes the MFMA
 // kernels (attn_fwd_d64.hip, attn_bwd_d64.hip); every other valid shape takes
-// the exact fp32 kernels in attn_generic.hip. There is no CPU path.
+// the fp32 kernels in attn_fp32.hip (or, for a backward launcher without
+// scratch, attn_generic.hip). There is no CPU path.
 #include <algorithm>
 #include <climits>
 #include <cstdio>
@@ -100,14 +101,15 @@ int fwd_impl(const float *q, const float *k, const float *v, float *o, float *ls
     err = dfattn::launch_fwd_d64(q, k, v, o, lse, (int)n_heads, (int)seq_len, scale, causal != 0,
                                  stream);
   else
-    err = dfattn::launch_fwd_generic(q, k, v, o, lse, (int)n_heads, (int)seq_len, (int)d_head,
-                                     scale, causal != 0, stream);
+    err = dfattn::launch_fwd_fp32(q, k, v, o, lse, (int)n_heads, (int)seq_len, (int)d_head, scale,
+                                  causal != 0, stream);
   return record_hip(err, "attention forward launch");
 }
 
 // Legacy backward: the caller's probability scratch (`capacity` floats) holds
-// O, lse and the fast path's workspace when it is large enough; otherwise the
-// self-contained generic kernel runs.
+// O, lse and the fast path's workspace when it is large enough, else lse and
+// Delta for the fp32 kernels (O goes through d_q, which their main launch
+// overwrites); without room for those the kernel that needs no scratch runs.
 int legacy_backward(const char *fn, const float *q, const float *k, const float *v,
                     const float *d_out, float *d_q, float *d_k, float *d_v, float *scratch,
                     size_t capacity, uint32_t n_heads, uint32_t seq_len, uint32_t d_head,
@@ -129,6 +131,13 @@ int legacy_backward(const char *fn, const float *q, const float *k, const float 
     if (err == hipSuccess)
       err = dfattn::launch_bwd_d64(q, k, v, o_ws, d_out, lse_ws, d_q, d_k, d_v, bwd_ws,
                                    (int)n_heads, (int)seq_len, scale, causal != 0, nullptr);
+  } else if (scratch != nullptr && aligned(scratch, alignof(float)) && 2 * (size_t)n_heads * seq_len <= capacity) {
+    float *lse_ws = scratch, *delta_ws = scratch + (size_t)n_heads * seq_len;
+    err = dfattn::launch_fwd_fp32(q, k, v, d_q, lse_ws, (int)n_heads, (int)seq_len, (int)d_head, scale,
+                                  causal != 0, nullptr);
+    if (err == hipSuccess)
+      err = dfattn::launch_bwd_fp32(q, k, v, d_q, d_out, lse_ws, delta_ws, d_q, d_k, d_v, (int)n_heads,
+                                    (int)seq_len, (int)d_head, scale, causal != 0, nullptr);
   } else {
     err = dfattn::launch_bwd_generic(q, k, v, d_out, d_q, d_k, d_v, (int)n_heads, (int)seq_len,
                                      (int)d_head, scale, causal != 0, nullptr);
@@ -372,8 +381,8 @@ int dfattn_bwd(const float *q, const float *k, const float *v, const float *o, c
     err = dfattn::launch_bwd_d64(q, k, v, o, d_o, lse, d_q, d_k, d_v, workspace, (int)n_heads,
                                  (int)seq_len, scale, causal != 0, s);
   else
-    err = dfattn::launch_bwd_generic(q, k, v, d_o, d_q, d_k, d_v, (int)n_heads, (int)seq_len,
-                                     (int)d_head, scale, causal != 0, s);
+    err = dfattn::launch_bwd_fp32(q, k, v, o, d_o, lse, static_cast<float *>(workspace), d_q, d_k, d_v,
+                                  (int)n_heads, (int)seq_len, (int)d_head, scale, causal != 0, s);
   return record_hip(err, "attention backward launch");
 }
 
@@ -405,7 +414,7 @@ int dfattn_bwd_preprocess(const float *q, const float *k, const float *v, const 
   if (st == DFATTN_OK) st = check_ptrs(fn, {q, k, v, o, d_o, lse});
   if (st == DFATTN_OK) st = check_workspace(fn, workspace, workspace_bytes, n_heads, seq_len, d_head);
   if (st != DFATTN_OK) return st;
-  // The generic kernel recomputes its row statistics itself: nothing to do.
+  // The fp32 backward needs no preparation beyond what its main phase does.
   if (!fast_path(d_head, {q, k, v, o, d_o})) return DFATTN_OK;
   if ((flags & ~(uint32_t)DFATTN_BWD_QKV_SAVED) != 0)
     return record_error(DFATTN_ERR_FLAGS, std::string(fn) + ": unknown flag bits");
@@ -430,8 +439,8 @@ int dfattn_bwd_main(const float *q, const float *k, const float *v, const float 
     err = dfattn::launch_bwd_main_d64(lse, d_q, d_k, d_v, workspace, (int)n_heads, (int)seq_len, scale,
                                       causal != 0, s);
   else
-    err = dfattn::launch_bwd_generic(q, k, v, d_o, d_q, d_k, d_v, (int)n_heads, (int)seq_len,
-                                     (int)d_head, scale, causal != 0, s);
+    err = dfattn::launch_bwd_fp32(q, k, v, o, d_o, lse, static_cast<float *>(workspace), d_q, d_k, d_v,
+                                  (int)n_heads, (int)seq_len, (int)d_head, scale, causal != 0, s);
   return record_hip(err, "attention backward launch");
 }
 
@@ -546,17 +555,17 @@ int dfattn_bwd_noalloc(const float *q, const float *k, const float *v, const flo
                             std::to_string((size_t)DFATTN_NOALLOC_SCRATCH_BYTES) + "); use dfattn_bwd");
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t err;
+  void *ws = nullptr;
+  st = scratch_on_current_device(fn, &ws);
+  if (st != DFATTN_OK) return st;
   if (fast_path(d_head, {q, k, v, o, d_o, lse, d_q, d_k, d_v})) {
-    void *ws = nullptr;
-    st = scratch_on_current_device(fn, &ws);
-    if (st != DFATTN_OK) return st;
     // Preprocess overwrites every workspace value the main kernel reads, so
     // nothing has to be cleared between calls.
     err = dfattn::launch_bwd_d64(q, k, v, o, d_o, lse, d_q, d_k, d_v, ws, (int)n_heads, (int)seq_len, scale,
                                  causal != 0, s);
   } else {
-    err = dfattn::launch_bwd_generic(q, k, v, d_o, d_q, d_k, d_v, (int)n_heads, (int)seq_len, (int)d_head,
-                                     scale, causal != 0, s);
+    err = dfattn::launch_bwd_fp32(q, k, v, o, d_o, lse, static_cast<float *>(ws), d_q, d_k, d_v, (int)n_heads,
+                                  (int)seq_len, (int)d_head, scale, causal != 0, s);
   }
   return record_hip(err, "attention backward launch");
 }

@@ -298,11 +298,16 @@ hipError_t launch_bwd_main_d64(const float *lse, float *d_q, float *d_k, float *
                                int n_heads, int seq_len, float scale, bool causal, hipStream_t stream,
                                int ldg = 0);
 
-// Generic fp32 kernels for any d_head in 1..=128 and any 4-byte alignment.
-// The backward recomputes everything it needs per row and uses no workspace.
-hipError_t launch_fwd_generic(const float *q, const float *k, const float *v, float *o,
-                              float *lse, int n_heads, int seq_len, int d_head, float scale,
-                              bool causal, hipStream_t stream);
+// fp32 kernels on the fp32 MFMA for any d_head in 1..=128 and any 4-byte
+// alignment (attn_fp32.hip). lse may be null in the forward. The backward takes
+// the forward's o and lse and `delta`, n_heads * seq_len floats of workspace.
+hipError_t launch_fwd_fp32(const float *q, const float *k, const float *v, float *o, float *lse, int n_heads,
+                           int seq_len, int d_head, float scale, bool causal, hipStream_t stream);
+hipError_t launch_bwd_fp32(const float *q, const float *k, const float *v, const float *o, const float *d_o,
+                           const float *lse, float *delta, float *d_q, float *d_k, float *d_v, int n_heads,
+                           int seq_len, int d_head, float scale, bool causal, hipStream_t stream);
+// The same backward from q, k, v and d_o alone, without any workspace
+// (attn_generic.hip): recomputes everything per row, adds dK and dV with atomics.
 hipError_t launch_bwd_generic(const float *q, const float *k, const float *v,
                               const float *d_o, float *d_q, float *d_k, float *d_v,
                               int n_heads, int seq_len, int d_head, float scale, bool causal,
