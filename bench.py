@@ -225,12 +225,12 @@ def short_kernel_name(name):
     for k in KERNELS + ("copyBuffer",):
         if k in name:
             return k
-    m = re.search(r"decode_d64_kernel(?:ILb([01])ELb([01])E|<(true|false), (true|false)>)", name)
+    m = re.search(r"decode_kernel(?:ILb([01])ELb([01])E|<(true|false), (true|false),)", name)
     if m:
         bf16 = m.group(1) == "1" or m.group(3) == "true"
         paged = m.group(2) == "1" or m.group(4) == "true"
-        return f"decode_d64_kernel<{'bf16' if bf16 else 'f32'}, {'paged' if paged else 'contiguous'}>"
-    for k in ("decode_reduce_kernel", "decode_generic_kernel"):
+        return f"decode_kernel<{'bf16' if bf16 else 'f32'}, {'paged' if paged else 'contiguous'}>"
+    for k in ("decode_reduce_kernel",):
         if k in name:
             return k
     return None

@@ -13,17 +13,19 @@
 // split-K layout (m, l: [H, n_chunks]; o: [H, n_chunks, D]), which
 // decode_reduce_kernel merges with the logsumexp identity.
 //
-// decode_d64_kernel (D = 64, the GPT-2 shape; fp32 or bf16 cache, contiguous
-// or paged): 8 waves; each wave takes 64-key groups. Its loads are coalesced
-// rows: lane l reads 4 values (16 bytes fp32, 8 bytes bf16) of row
-// 4j + l/16 of the group at column 4*(l%16), for j = 0..15, K and V alike.
-// The score of a row is reduced over its 16 lanes, gathered through LDS so
-// that lane r holds key r for the softmax, and P goes back through LDS to
-// the V lanes. decode_generic_kernel handles every other D (1..128): one wave
-// per workgroup, lanes over d, one key at a time.
+// decode_kernel: 8 waves; each wave takes groups of keys. Its loads are coalesced
+// rows: LPR lanes (8, 16 or 32, the smallest power of two >= D/4) read 4 values
+// each (16 bytes fp32, 8 bytes bf16) of one row, 64/LPR rows per load, all of a
+// group's K and V loads before the first wait. The score of a row is reduced
+// over its lanes, gathered through LDS so that lane r holds key r for the
+// softmax, and P goes back through LDS to the V lanes. Rows that are not 4-value
+// aligned (D % 4 != 0, or an odd base) load value by value.
 #include "dfattn_internal.h"
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
 
 namespace dfattn {
 namespace {
@@ -47,10 +49,6 @@ struct DecodeArgs {
 __device__ __forceinline__ size_t cache_row(const DecodeArgs &a, int t) {
   if (a.table == nullptr) return (size_t)t;
   return (size_t)a.table[t / a.page_size] * (size_t)a.page_size + (size_t)(t % a.page_size);
-}
-
-__device__ __forceinline__ float bf16_bits_to_float(unsigned short b) {
-  return __builtin_bit_cast(float, (unsigned)b << 16);
 }
 
 // 4 consecutive values of a cache row: the raw bits (fp32: the floats; bf16:
@@ -82,23 +80,41 @@ __device__ __forceinline__ float4 widen4(uint4 r) {
     return __builtin_bit_cast(float4, r);
 }
 
-// Sum over each row of 16 lanes, in every lane of the row: DPP rotations
-// within the row (row_ror:8, 4, 2, 1), full-rate VALU instead of LDS-pipe
-// permutes.
-__device__ __forceinline__ float row16_sum(float x) {
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x124, 0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x122, 0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x121, 0xf, 0xf, false));
-  return x;
+// The same for rows without that alignment: value by value, the values at or
+// past D (clamped loads) zeroed in widen4_any.
+template <bool BF16>
+__device__ __forceinline__ uint4 load4_any(const void *base, size_t row, int d0, int D) {
+  unsigned u[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const size_t e = row + min(d0 + j, D - 1);
+    u[j] = BF16 ? (unsigned)reinterpret_cast<const unsigned short *>(base)[e] << 16
+                : reinterpret_cast<const unsigned *>(base)[e];
+  }
+  return make_uint4(u[0], u[1], u[2], u[3]);
+}
+__device__ __forceinline__ float4 widen4_any(uint4 r, int d0, int D) {
+  const float4 v = __builtin_bit_cast(float4, r);
+  return make_float4(d0 < D ? v.x : 0.f, d0 + 1 < D ? v.y : 0.f, d0 + 2 < D ? v.z : 0.f, d0 + 3 < D ? v.w : 0.f);
 }
 
-template <bool BF16>
-__device__ __forceinline__ float load1(const void *base, size_t elem) {
-  if constexpr (BF16)
-    return bf16_bits_to_float(reinterpret_cast<const unsigned short *>(base)[elem]);
-  else
-    return reinterpret_cast<const float *>(base)[elem];
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float x) {
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+}
+// Sum over each aligned group of LPR lanes, in every lane of the group: DPP
+// moves within the row of 16 lanes (rotations by 8, 4, 2, 1, or for 8 lanes
+// two swaps within the quad and the half-row mirror), full-rate VALU instead
+// of LDS-pipe permutes, and for 32 lanes one permlane16 swap.
+template <int LPR>
+__device__ __forceinline__ float group_sum(float x) {
+  if constexpr (LPR == 8) return add_dpp<0x141>(add_dpp<0x4e>(add_dpp<0xb1>(x)));
+  x = add_dpp<0x121>(add_dpp<0x122>(add_dpp<0x124>(add_dpp<0x128>(x))));
+  if constexpr (LPR == 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return x;
 }
 
 // Writes one chunk's (m, l, o) — m and the scores in the log2 domain — as the
@@ -119,135 +135,167 @@ __device__ __forceinline__ void write_chunk(const DecodeArgs &a, int h, int c, i
   }
 }
 
-template <bool BF16, bool PAGED>
-__global__ __launch_bounds__(kDecThreads) void decode_d64_kernel(DecodeArgs a) {
-  __shared__ float s_lds[kDecWaves][64];   // scores, then P, of the wave's group
-  __shared__ unsigned row_lds[kDecWaves][64];  // paged: the group's physical rows
+// How a row lies on its lanes: it fills them (D = 4 * LPR), it leaves some out,
+// or its 4-value pieces are not aligned (any D).
+enum Rows { kFull, kPartial, kUnaligned };
+
+// Bound by HBM (K and V are read once) or, for short caches, by latency: one
+// group's loads are all in flight before its first wait. Against one wave per
+// chunk taking one key at a time, any D but 64 (H, keys): 274 -> 4.5 us (4, 509,
+// D 32 bf16 paged), 368 -> 10.6 us (7, 18490, D 32 bf16 paged), 527 -> 14 us (8,
+// 4096, D 128 fp32), 7.0 ms -> 395 us (16, 131072, D 128 fp32: 5.4 TB/s).
+// Row and key bounds checked at run time in every group cost a 1024-key decode
+// 0.8 of 8.0 us: D = 32, 64 and 128 have kernels of their own, and only the
+// last group of a chunk has key bounds.
+template <bool BF16, bool PAGED, int LPR, Rows ROWS>
+__global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeArgs a) {
+  constexpr int kRowsPerLoad = 64 / LPR;
+  constexpr int kLoads = LPR == 8 ? 8 : 16;           // K (and V) loads per group and lane
+  constexpr int kGroup = kRowsPerLoad * kLoads;       // keys per group: 64, 64, 32
+  constexpr int kCols = 4 * LPR;
+  constexpr bool VEC = ROWS != kUnaligned;
+  // Physical rows of 32-bit size but for the narrowest rows, which a GPU could hold more of.
+  using row_t = std::conditional_t<LPR == 8, size_t, unsigned>;
+  __shared__ float s_lds[kDecWaves][kGroup];   // scores, then P, of the wave's group
+  __shared__ row_t row_lds[kDecWaves][kGroup];  // paged: the group's physical rows
   __shared__ float m_lds[kDecWaves], l_lds[kDecWaves];
-  __shared__ float o_lds[kDecWaves][64];
+  __shared__ __attribute__((aligned(16))) float o_lds[kDecWaves][kCols];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int sub = lane >> 4, dq = lane & 15;  // row 4j + sub of a group, columns 4*dq .. +3
-  const int h = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
-  const int t0 = c * a.chunk, t1 = min(a.L, t0 + a.chunk);
-  const size_t dm = (size_t)a.H * 64;
-  const size_t col = (size_t)h * 64 + 4 * dq;
-  const float4 q4 = *reinterpret_cast<const float4 *>(a.q + col);
+  const int sub = lane / LPR, d0 = 4 * (lane % LPR);  // row kRowsPerLoad*j + sub of a group, columns d0 .. +3
+  const int h = blockIdx.y;
+  const int D = ROWS == kFull ? kCols : a.D;
+  const size_t dm = (size_t)a.H * D, hoff = (size_t)h * D;
+  // Lanes past the row's values read column 0 and add nothing.
+  const bool on = d0 < D;
+  const size_t col = hoff + (on ? d0 : 0);
+  float4 q4;
+  if constexpr (VEC)
+    q4 = *reinterpret_cast<const float4 *>(a.q + col);
+  else
+    q4 = widen4_any(load4_any<false>(a.q, hoff, d0, D), d0, D);
   const float c2 = a.scale * kLog2e;
 
-  float m = -INFINITY, l = 0.f;
-  float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int g0 = t0 + 64 * wave; g0 < t1; g0 += 64 * kDecWaves) {
-    // This wave's group: keys g0 .. g0+63 (those below t1). Paged: lane r
-    // looks up the physical row of key g0 + r once, for every lane.
-    if constexpr (PAGED) {
-      const int t = min(g0 + lane, t1 - 1);
-      row_lds[wave][lane] = (unsigned)cache_row(a, t);
+  for (int c = blockIdx.x;;) {
+    const int t0 = c * a.chunk, t1 = min(a.L, t0 + a.chunk);
+    float m = -INFINITY, l = 0.f;
+    float4 o4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    // One group: keys g0 .. g0+kGroup-1, the last group's only those below t1.
+    auto group = [&](int g0, auto last) {
+      constexpr bool kLast = decltype(last)::value;
+      const int n = kLast ? t1 - g0 : kGroup;
+      // Paged: lane r looks up the physical row of key g0 + r once, for every lane.
+      if constexpr (PAGED) {
+        if (lane < kGroup) row_lds[wave][lane] = (row_t)cache_row(a, g0 + (kLast ? min(lane, n - 1) : lane));
+        __builtin_amdgcn_wave_barrier();
+      }
+      // Rows past the last key read its row instead, so every load is unconditional.
+      uint4 kr[kLoads], vr[kLoads];
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        int r = kRowsPerLoad * j + sub;
+        if (kLast) r = min(r, n - 1);
+        const size_t row = PAGED ? (size_t)row_lds[wave][r] : (size_t)(g0 + r);
+        if constexpr (VEC) {
+          kr[j] = load4_raw<BF16>(a.k, row * dm + col);
+          vr[j] = load4_raw<BF16>(a.v, row * dm + col);
+        } else {
+          kr[j] = load4_any<BF16>(a.k, row * dm + hoff, d0, D);
+          vr[j] = load4_any<BF16>(a.v, row * dm + hoff, d0, D);
+        }
+      }
+      auto widen = [&](uint4 x) {
+        if constexpr (VEC)
+          return widen4<BF16>(x);
+        else
+          return widen4_any(x, d0, D);
+      };
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        const float4 k4 = widen(kr[j]);
+        const float part = q4.x * k4.x + q4.y * k4.y + q4.z * k4.z + q4.w * k4.w;
+        const float s = group_sum<LPR>(on ? part : 0.f);
+        if (d0 == 0) s_lds[wave][kRowsPerLoad * j + sub] = s;
+      }
       __builtin_amdgcn_wave_barrier();
+      // Online softmax over the group, lane r = key g0 + r.
+      const bool valid = lane < kGroup && (!kLast || lane < n);
+      const float s2 = valid ? s_lds[wave][lane % kGroup] * c2 : -INFINITY;
+      const float m_new = fmaxf(m, wave_max(s2));
+      const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+      const float p = valid ? __builtin_amdgcn_exp2f(s2 - m_new) : 0.f;
+      l = l * alpha + p;
+      m = m_new;
+      __builtin_amdgcn_wave_barrier();
+      if (lane < kGroup) s_lds[wave][lane] = p;
+      __builtin_amdgcn_wave_barrier();
+      o4.x *= alpha;
+      o4.y *= alpha;
+      o4.z *= alpha;
+      o4.w *= alpha;
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        // (Rows past the last key are left out, not weighted by 0: its value may be infinite.)
+        if (kLast && kRowsPerLoad * j + sub >= n) continue;
+        const float pj = s_lds[wave][kRowsPerLoad * j + sub];
+        const float4 v4 = widen(vr[j]);
+        o4.x += pj * v4.x;
+        o4.y += pj * v4.y;
+        o4.z += pj * v4.z;
+        o4.w += pj * v4.w;
+      }
+      __builtin_amdgcn_wave_barrier();
+    };
+    int g0 = t0 + kGroup * wave;
+    for (; g0 + kGroup <= t1; g0 += kGroup * kDecWaves) group(g0, std::false_type{});
+    if (g0 < t1) group(g0, std::true_type{});
+
+    // The wave's (m, l, o): l summed over lanes, o over the rows of a load.
+    l = wave_sum(l);
+#pragma unroll
+    for (int off = LPR; off < 64; off <<= 1) {
+      o4.x += __shfl_xor(o4.x, off, 64);
+      o4.y += __shfl_xor(o4.y, off, 64);
+      o4.z += __shfl_xor(o4.z, off, 64);
+      o4.w += __shfl_xor(o4.w, off, 64);
     }
-    // Rows past t1 read row t1-1 instead (their P is 0), so every load is
-    // unconditional.
-    uint4 kr[16], vr[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int t = min(g0 + 4 * j + sub, t1 - 1);
-      const size_t row = PAGED ? (size_t)row_lds[wave][min(4 * j + sub, t1 - 1 - g0)] : (size_t)t;
-      const size_t e = row * dm + col;
-      kr[j] = load4_raw<BF16>(a.k, e);
-      vr[j] = load4_raw<BF16>(a.v, e);
+    if (lane == 0) {
+      m_lds[wave] = m;
+      l_lds[wave] = l;
     }
+    if (sub == 0) *reinterpret_cast<float4 *>(&o_lds[wave][d0]) = o4;
+    __syncthreads();
+    if (tid < kCols && tid < D) {
+      // Merge the waves (a wave with no keys has m = -inf and weight 0).
+      float mm = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float4 k4 = widen4<BF16>(kr[j]);
-      const float s = row16_sum(q4.x * k4.x + q4.y * k4.y + q4.z * k4.z + q4.w * k4.w);
-      if (dq == 0) s_lds[wave][4 * j + sub] = s;
+      for (int w = 0; w < kDecWaves; ++w) mm = fmaxf(mm, m_lds[w]);
+      float ll = 0.f, oo = 0.f;
+#pragma unroll
+      for (int w = 0; w < kDecWaves; ++w) {
+        const float f = m_lds[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_lds[w] - mm);
+        ll += f * l_lds[w];
+        oo += f * o_lds[w][tid];
+      }
+      write_chunk(a, h, c, tid, mm, ll, oo);
     }
-    __builtin_amdgcn_wave_barrier();
-    // Online softmax over the group, lane r = key g0 + r.
-    const bool valid = g0 + lane < t1;
-    const float s2 = valid ? s_lds[wave][lane] * c2 : -INFINITY;
-    const float m_new = fmaxf(m, wave_max(s2));
-    const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
-    const float p = valid ? __builtin_amdgcn_exp2f(s2 - m_new) : 0.f;
-    l = l * alpha + p;
-    m = m_new;
-    __builtin_amdgcn_wave_barrier();
-    s_lds[wave][lane] = p;
-    __builtin_amdgcn_wave_barrier();
-    o4.x *= alpha;
-    o4.y *= alpha;
-    o4.z *= alpha;
-    o4.w *= alpha;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float pj = s_lds[wave][4 * j + sub];
-      const float4 v4 = widen4<BF16>(vr[j]);
-      o4.x += pj * v4.x;
-      o4.y += pj * v4.y;
-      o4.z += pj * v4.z;
-      o4.w += pj * v4.w;
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
-  // The wave's (m, l, o): l summed over lanes, o over the four row groups.
-  l = wave_sum(l);
-#pragma unroll
-  for (int off = 16; off < 64; off <<= 1) {
-    o4.x += __shfl_xor(o4.x, off, 64);
-    o4.y += __shfl_xor(o4.y, off, 64);
-    o4.z += __shfl_xor(o4.z, off, 64);
-    o4.w += __shfl_xor(o4.w, off, 64);
-  }
-  if (lane == 0) {
-    m_lds[wave] = m;
-    l_lds[wave] = l;
-  }
-  if (sub == 0) *reinterpret_cast<float4 *>(&o_lds[wave][4 * dq]) = o4;
-  __syncthreads();
-  if (wave == 0) {
-    // Merge the waves (a wave with no keys has m = -inf and weight 0).
-    float mm = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kDecWaves; ++w) mm = fmaxf(mm, m_lds[w]);
-    float ll = 0.f, oo = 0.f;
-#pragma unroll
-    for (int w = 0; w < kDecWaves; ++w) {
-      const float f = m_lds[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_lds[w] - mm);
-      ll += f * l_lds[w];
-      oo += f * o_lds[w][lane];
-    }
-    write_chunk(a, h, c, lane, mm, ll, oo);
+    // Another chunk only where a grid cannot hold them all.
+    c += gridDim.x;
+    if (c >= a.n_chunks) break;
+    __syncthreads();
   }
 }
 
-// Any D in 1..128: one wave per workgroup, lane d holds columns d and d+64,
-// keys one at a time (the reference's order of work, wave64 wide).
-template <bool BF16>
-__global__ __launch_bounds__(64) void decode_generic_kernel(DecodeArgs a) {
-  const int lane = threadIdx.x;
-  const int h = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
-  const int t0 = c * a.chunk, t1 = min(a.L, t0 + a.chunk);
-  const int D = a.D;
-  const size_t dm = (size_t)a.H * D, hoff = (size_t)h * D;
-  const bool in0 = lane < D, in1 = lane + 64 < D;
-  const float q0 = in0 ? a.q[hoff + lane] : 0.f, q1 = in1 ? a.q[hoff + lane + 64] : 0.f;
-  const float c2 = a.scale * kLog2e;
-  float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int t = t0; t < t1; ++t) {
-    const size_t base = cache_row(a, t) * dm + hoff;
-    float s = 0.f;
-    if (in0) s += q0 * load1<BF16>(a.k, base + lane);
-    if (in1) s += q1 * load1<BF16>(a.k, base + lane + 64);
-    s = wave_sum(s) * c2;
-    const float m_new = fmaxf(m, s);
-    const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
-    const float p = __builtin_amdgcn_exp2f(s - m_new);
-    l = l * alpha + p;
-    m = m_new;
-    o0 = o0 * alpha + (in0 ? p * load1<BF16>(a.v, base + lane) : 0.f);
-    o1 = o1 * alpha + (in1 ? p * load1<BF16>(a.v, base + lane + 64) : 0.f);
-  }
-  if (in0) write_chunk(a, h, c, lane, m, l, o0);
-  if (in1) write_chunk(a, h, c, lane + 64, m, l, o1);
+template <int LPR, Rows ROWS>
+void launch_decode_rows(const DecodeArgs &a, bool bf16, dim3 grid, hipStream_t stream) {
+  const bool paged = a.table != nullptr;
+  if (bf16 && paged)
+    hipLaunchKernelGGL((decode_kernel<true, true, LPR, ROWS>), grid, dim3(kDecThreads), 0, stream, a);
+  else if (bf16)
+    hipLaunchKernelGGL((decode_kernel<true, false, LPR, ROWS>), grid, dim3(kDecThreads), 0, stream, a);
+  else if (paged)
+    hipLaunchKernelGGL((decode_kernel<false, true, LPR, ROWS>), grid, dim3(kDecThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((decode_kernel<false, false, LPR, ROWS>), grid, dim3(kDecThreads), 0, stream, a);
 }
 
 // Merges the split-K partials of one head (attention_fused.cu:712-757):
@@ -340,7 +388,7 @@ __global__ __launch_bounds__(kRedThreads) void decode_reduce_kernel(const float 
 hipError_t launch_decode(const float *q, const void *k, const void *v, const int32_t *block_table,
                          int page_size, bool bf16, float *out, float *lse, int n_heads, int cur_len,
                          int d_head, float scale, int chunk, float *part_m, float *part_l, float *part_o,
-                         bool fast, hipStream_t stream) {
+                         bool aligned, hipStream_t stream) {
   DecodeArgs a;
   a.q = q;
   a.k = k;
@@ -358,23 +406,23 @@ hipError_t launch_decode(const float *q, const void *k, const void *v, const int
   a.part_m = part_m;
   a.part_l = part_l;
   a.part_o = part_o;
-  const unsigned grid = (unsigned)(n_heads * a.n_chunks);
-  if (fast && d_head == 64) {
-    const bool paged = block_table != nullptr;
-    if (bf16 && paged)
-      hipLaunchKernelGGL((decode_d64_kernel<true, true>), dim3(grid), dim3(kDecThreads), 0, stream, a);
-    else if (bf16)
-      hipLaunchKernelGGL((decode_d64_kernel<true, false>), dim3(grid), dim3(kDecThreads), 0, stream, a);
-    else if (paged)
-      hipLaunchKernelGGL((decode_d64_kernel<false, true>), dim3(grid), dim3(kDecThreads), 0, stream, a);
+  const dim3 grid((unsigned)std::min(a.n_chunks, 1 << 20), (unsigned)n_heads);
+  // 8 lanes to a row up to 32 values, 16 up to 64, 32 up to 128.
+  auto with_lanes = [&](auto lpr) {
+    constexpr int LPR = decltype(lpr)::value;
+    if (!aligned)
+      launch_decode_rows<LPR, kUnaligned>(a, bf16, grid, stream);
+    else if (d_head == 4 * LPR)
+      launch_decode_rows<LPR, kFull>(a, bf16, grid, stream);
     else
-      hipLaunchKernelGGL((decode_d64_kernel<false, false>), dim3(grid), dim3(kDecThreads), 0, stream, a);
-  } else {
-    if (bf16)
-      hipLaunchKernelGGL(decode_generic_kernel<true>, dim3(grid), dim3(64), 0, stream, a);
-    else
-      hipLaunchKernelGGL(decode_generic_kernel<false>, dim3(grid), dim3(64), 0, stream, a);
-  }
+      launch_decode_rows<LPR, kPartial>(a, bf16, grid, stream);
+  };
+  if (d_head <= 32)
+    with_lanes(std::integral_constant<int, 8>{});
+  else if (d_head <= 64)
+    with_lanes(std::integral_constant<int, 16>{});
+  else
+    with_lanes(std::integral_constant<int, 32>{});
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || a.n_chunks == 1) return err;
   hipLaunchKernelGGL(decode_reduce_kernel, dim3((unsigned)n_heads), dim3(kRedThreads), 0, stream, part_m, part_l,

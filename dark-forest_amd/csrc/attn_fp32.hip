@@ -54,15 +54,6 @@ __device__ __forceinline__ float column_sum(float v) {
   return pair_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
-// Grids of any number of workgroups as (x, y) with x <= 2^22 (the work items
-// of a grid's x must stay below 2^32); the last row may hold workgroups past
-// the total.
-constexpr unsigned kGridX = 1u << 22;
-inline dim3 linear_grid(size_t total) {
-  return total <= kGridX ? dim3((unsigned)total) : dim3(kGridX, (unsigned)((total + kGridX - 1) / kGridX));
-}
-__device__ __forceinline__ unsigned linear_block() { return blockIdx.y * kGridX + blockIdx.x; }
-
 // One [S, H*D] operand as seen by a head.
 struct Shape {
   int S, D, ld, hoff;

@@ -183,9 +183,9 @@ int check_decode(const char *fn, const float *q, const void *k, const void *v, c
   return DFATTN_OK;
 }
 
-bool decode_fast(uint32_t d_head, bool bf16, const float *q, const void *k, const void *v) {
+bool decode_aligned(uint32_t d_head, bool bf16, const float *q, const void *k, const void *v) {
   const size_t kv_align = bf16 ? 8 : 16;
-  return d_head == 64 && aligned(q, 16) && aligned(k, kv_align) && aligned(v, kv_align);
+  return d_head % 4 == 0 && aligned(q, 16) && aligned(k, kv_align) && aligned(v, kv_align);
 }
 
 // The reference's decode launchers: null stream, errors recorded for
@@ -205,7 +205,7 @@ int legacy_decode(const char *fn, const float *q, const void *k, const void *v, 
   const hipError_t err = dfattn::launch_decode(
       q, k, v, paged ? table : nullptr, (int)page_size, bf16, out, nullptr, (int)n_heads, (int)cur_len,
       (int)d_head, scale, split ? (int)chunk : (int)cur_len, split ? pm : nullptr, split ? pl : nullptr,
-      split ? po : nullptr, decode_fast(d_head, bf16, q, k, v), nullptr);
+      split ? po : nullptr, decode_aligned(d_head, bf16, q, k, v), nullptr);
   return record_hip(err, fn);
 }
 
@@ -675,7 +675,7 @@ int dfattn_decode(const float *q, const void *k_cache, const void *v_cache, cons
   const hipError_t err = dfattn::launch_decode(
       q, k_cache, v_cache, block_table, (int)(paged ? page_size : 1), bf16, out, lse, (int)n_heads,
       (int)cur_seq_len, (int)d_head, scale, (int)chunk, pm, pl, po,
-      decode_fast(d_head, bf16, q, k_cache, v_cache) && (lse == nullptr || aligned(lse, 4)),
+      decode_aligned(d_head, bf16, q, k_cache, v_cache),
       static_cast<hipStream_t>(stream));
   return record_hip(err, "decode launch");
 }

@@ -90,6 +90,15 @@ __device__ __forceinline__ int uniform_clamp0(int x) {
 }
 constexpr float kLn2 = 0.6931471805599453f;
 
+// Grids of any number of workgroups as (x, y) with x <= 2^22 (the work items
+// of a grid's x must stay below 2^32); the last row may hold workgroups past
+// the total.
+constexpr unsigned kGridX = 1u << 22;
+inline dim3 linear_grid(size_t total) {
+  return total <= kGridX ? dim3((unsigned)total) : dim3(kGridX, (unsigned)((total + kGridX - 1) / kGridX));
+}
+__device__ __forceinline__ unsigned linear_block() { return blockIdx.y * kGridX + blockIdx.x; }
+
 // D = 64 fast path: one 32x32x16 fp16 MFMA (fp32 accumulate). Operand
 // convention used by every kernel here: for A (M x K) lane l holds row
 // m = l % 32 and the 8 contraction slots k = 8*(l/32) + j, j = 0..7; for B
@@ -319,12 +328,12 @@ hipError_t launch_bwd_generic(const float *q, const float *k, const float *v,
 // head writes out (and lse if not null) directly; otherwise the key range is
 // split into ceil(cur_len / chunk) chunks whose partials (part_m, part_l:
 // [n_heads, n_chunks], part_o: [n_heads, n_chunks, d_head]) a second kernel
-// merges. fast: d_head == 64 with 16-byte aligned q and 8-byte aligned
-// cache rows may take the coalesced kernel. cur_len >= 1.
+// merges. aligned: four consecutive values of a row (d_head % 4 == 0) start at
+// a multiple of their size in q, k and v. cur_len >= 1.
 hipError_t launch_decode(const float *q, const void *k, const void *v, const int32_t *block_table,
                          int page_size, bool bf16, float *out, float *lse, int n_heads, int cur_len,
                          int d_head, float scale, int chunk, float *part_m, float *part_l, float *part_o,
-                         bool fast, hipStream_t stream);
+                         bool aligned, hipStream_t stream);
 
 // Elementwise companions of the decode path (attn_aux.hip). trained >= 1.
 hipError_t launch_pos_embed_interpolate(const float *table, float *out, unsigned pos, unsigned trained,
