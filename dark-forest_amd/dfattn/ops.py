@@ -181,7 +181,7 @@ def _ids_ptr(t):
     torch = _torch()
     if not t.is_cuda or t.dtype != torch.int32 or not t.is_contiguous():
         raise ValueError("token ids must be a contiguous int32 device tensor")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def logit_ce_chunk(logits, targets, grad, row_loss, total_rows):
