@@ -27,6 +27,7 @@
 // — the row statistic the backward recomputes P from.
 #include "dfattn_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace dfattn {
@@ -604,6 +605,223 @@ __global__ __launch_bounds__(kThreads) void fwd_d64_kernel(
   }
 }
 
+// ---------------------------------------------------------- short sequences
+// The kernel above takes 128 query rows a workgroup and 0.57 us for each 64-key
+// tile: at S = 1024 its 8 workgroups per head leave most of the 256 CUs idle
+// and the longest walks 16 tiles. Here a workgroup of four waves takes 32 query
+// rows, and its waves take the 32-key tiles w, w + 4, ... on their own, each
+// through LDS tiles of its own and without barriers until they merge: four
+// times the workgroups and a quarter of the serial length. Every workgroup
+// fetches and rounds the K and V rows it reads, 16 KB for 32 x 32 scores, so
+// what bounds it is L2 to L1 (256 cycles of a CU a tile); longer sequences are
+// better off with tiles shared by 128 rows. Same operands and roundings (scaled
+// Q, K, V and P in fp16, fp32 sums).
+constexpr int kShortWaves = 4;
+constexpr int kShortRows = 32;
+
+__global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
+    const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float *__restrict__ O,
+    float *__restrict__ LSE, int H, int S, float qscale, int causal, int n_blocks, int fold,
+    half_t *__restrict__ Q16, half_t *__restrict__ K16, half_t *__restrict__ V16, half_t *__restrict__ QLO,
+    int qlo_stride, int ldi) {
+  // Per wave: its K and V tiles, [32][64] fp16 each; at the end its 32 result
+  // registers, as [4][2][64] float4.
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kShortWaves][8 * 64 * 16];
+  __shared__ float m_lds[kShortWaves][kShortRows], l_lds[kShortWaves][kShortRows];
+  const int lane = threadIdx.x & 63, c = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int idx = __builtin_amdgcn_readfirstlane(blockIdx.x / H), head = blockIdx.x - idx * H;
+  const int hoff = head * kD, ld = H * kD;
+  // Longest blocks first under causal masking; with `fold` the second half of
+  // the workgroups takes the short blocks in ascending order.
+  const int n_long = (n_blocks + 1) / 2;
+  const int blk = !causal ? idx : fold && idx >= n_long ? idx - n_long : n_blocks - 1 - idx;
+  const int q0 = blk * kShortRows;
+  const int n_tiles = ((causal ? min(S, q0 + kShortRows) : S) + kShortRows - 1) / kShortRows;
+  const int query = q0 + c;
+  const int key_lim = causal ? min(query, S - 1) : S - 1;
+  const bool save = Q16 != nullptr;
+
+  // Rows of tile t (32 rows) of X; rows past S read as zeros. (n_heads <= 65535
+  // and row strides <= 2^22: 32 rows span less than 2^31 bytes.)
+  auto tile = [&](const float *X, int t) {
+    const int rows = uniform_clamp0<kShortRows>(S - t * kShortRows);
+    return buffer_rsrc(X + (size_t)min(t * kShortRows, S) * ldi + hoff,
+                       rows > 0 ? (unsigned)((rows - 1) * ldi + kD) * 4u : 0u);
+  };
+  auto load4 = [](auto rs, int off) {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+  };
+  // A tile by full rows: load i holds values 4*(lane%16) .. +3 of row 4i + lane/16.
+  const int lrow = lane >> 4, lcol = 4 * (lane & 15);
+  auto load_tile = [&](const float *X, int t, float4 (&x)[8]) {
+    const auto rs = tile(X, t);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = load4(rs, ((4 * i + lrow) * ldi + lcol) * 4);
+  };
+  half_t *kt = reinterpret_cast<half_t *>(lds_raw[wave]), *vt = kt + kShortRows * kD;
+  int soff[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) soff[i] = tile_off(4 * i + lrow, lcol);
+  // Row c, values 16*ds + 8*hh + 0..7, of an LDS tile.
+  auto read_rows = [&](const half_t *tl, half8_t (&x)[4]) {
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) x[ds] = *reinterpret_cast<const half8_t *>(tl + tile_off(c, 8 * (2 * ds + hh)));
+  };
+  // fp16 copies for the backward (its rounding) and the residues of rows 0-63,
+  // from a tile's loads: rows 4i + lrow of tile t.
+  auto save4 = [&](half_t *dst16, int lo_tile, int t, int i, half4_t x, float4 raw, float scale) {
+    const int row = t * kShortRows + 4 * i + lrow;
+    if (row >= S) return;
+    *reinterpret_cast<half4_t *>(dst16 + ((size_t)head * S + row) * kD + lcol) = x;
+    if (lo_tile >= 0 && row < kLoRows)
+      *reinterpret_cast<half4_t *>(QLO + (size_t)head * qlo_stride + (lo_tile * kLoRows + row) * kD + lcol) =
+          scaled_residue4(raw, scale);
+  };
+
+  half8_t qf[4];
+  float4 kr[8], vr[8];
+  {
+    float4 qr[8];
+    load_tile(Q, blk, qr);
+    load_tile(K, wave, kr);
+    load_tile(V, wave, vr);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const half4_t x = round_scaled4(qr[i], qscale);
+      *reinterpret_cast<half4_t *>(kt + soff[i]) = x;
+      if (save && (i >> 1) == wave) save4(Q16, 0, blk, i, x, qr[i], qscale);
+    }
+    read_rows(kt, qf);
+  }
+
+  f32x16 o[2];
+  o[0] = o[1] = f32x16{};
+  float m = -INFINITY, l = 0.f;
+  f32x16 negm = f32x16{};  // -m in every register (0 while m = -inf)
+  for (int t = wave; t < n_tiles; t += kShortWaves) {
+    const bool own = save && t == blk;  // the tile of the workgroup's own rows
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const half4_t kx = to_half4(kr[i]), vx = to_half4(vr[i]);
+      *reinterpret_cast<half4_t *>(kt + soff[i]) = kx;
+      *reinterpret_cast<half4_t *>(vt + soff[i]) = vx;
+      if (own) {
+        save4(K16, 1, t, i, kx, kr[i], 1.f);
+        save4(V16, -1, t, i, vx, vr[i], 1.f);
+      }
+    }
+    load_tile(K, t + kShortWaves, kr);
+    load_tile(V, t + kShortWaves, vr);
+    half8_t kf[4];
+    read_rows(kt, kf);
+    f32x16 s = mfma32x32x16(kf[0], qf[0], negm);
+#pragma unroll
+    for (int ds = 1; ds < 4; ++ds) s = mfma32x32x16(kf[ds], qf[ds], s);
+    const int k0 = t * kShortRows;
+    if (k0 + kShortRows - 1 > (causal ? q0 : S - 1)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + 8 * (r >> 2) + 4 * hh + (r & 3) > key_lim) s[r] = -INFINITY;
+    }
+    half8_t pf[2];
+    auto probs = [&] {
+      float a = 0.f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pf[j][i] = (half_t)fast_exp2(s[8 * j + i]);
+        a = sum8_f16(pf[j], a);
+      }
+      return a;
+    };
+    // As in the staged kernel: the reference point moves only when a sum of P
+    // reaches 2^8 (or none is set yet).
+    float psum = probs();
+    if (__any(psum >= kRescaleSum || m == -INFINITY)) {
+      float mx = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = pair_max(mx);
+      if (__any(mx > kRescale || m == -INFINITY)) {
+        const float m_use = m == -INFINITY ? 0.f : m;
+        const float m_new = fmaxf(m, m_use + mx);
+        const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - m_new);
+        const float shift = m_new == -INFINITY ? 0.f : m_new - m_use;
+        l *= alpha;
+        o[0] *= alpha;
+        o[1] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          s[r] -= shift;
+          negm[r] -= shift;
+        }
+        m = m_new == -INFINITY ? m_new : -negm[0];
+        psum = probs();
+      }
+    }
+    l += psum;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) o[db] = mfma32x32x16(tile_tr8(vt, ks, db, lane), pf[ks], o[db]);
+  }
+
+  // Merge: each wave writes (m, l, O) (over its own tiles); wave w finishes
+  // registers 4w .. 4w+3 of both blocks, values 32*db + 8w + 4*hh + 0..3.
+  const float lsum = pair_sum(l);
+  if (hh == 0) {
+    m_lds[wave][c] = m;
+    l_lds[wave][c] = lsum;
+  }
+  f32x4 *part = reinterpret_cast<f32x4 *>(lds_raw[wave]);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+      part[(2 * g + db) * 64 + lane] = f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+  __syncthreads();
+  float top = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kShortWaves; ++w) top = fmaxf(top, m_lds[w][c]);
+  const float use = top == -INFINITY ? 0.f : top;
+  float sum = 0.f;
+  f32x4 res[2] = {};
+#pragma unroll
+  for (int w = 0; w < kShortWaves; ++w) {
+    const float a = fast_exp2(m_lds[w][c] - use);
+    const f32x4 *p = reinterpret_cast<const f32x4 *>(lds_raw[w]);
+    sum += a * l_lds[w][c];
+#pragma unroll
+    for (int db = 0; db < 2; ++db) res[db] += a * p[(2 * wave + db) * 64 + lane];
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+  if (query < S) {
+    float *dst = O + (size_t)query * ld + hoff + 8 * wave + 4 * hh;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+      *reinterpret_cast<float4 *>(dst + 32 * db) =
+          make_float4(res[db][0] * inv, res[db][1] * inv, res[db][2] * inv, res[db][3] * inv);
+    if (LSE != nullptr && wave == 0 && hh == 0)
+      LSE[(size_t)head * S + query] = sum > 0.f ? (top + log2f(sum)) * kLn2 : -INFINITY;
+  }
+}
+
+// Which forward: both times estimated from what they measured, in ns above
+// their common fixed 4 us. The short kernel: 200 ns of one CU a 32 x 32 tile over
+// 256 CUs, but at least 620 ns for each of a wave's tiles in turn; the staged
+// one: 566 ns for each 64-key tile of its longest workgroup (when all of them
+// run at once; longer otherwise, and then the short kernel has lost anyway).
+// Measured, short against staged, us: H = 12 causal S = 128 5.0 / 7.1, 512 7.4 /
+// 10.0, 1024 11.4 / 14.1, 1536 15.7 / 17.8, 2048 25.3 / 22.7 (staged); unmasked
+// 512 7.6 / 11.6, 1536 28.8 / 19.8 (staged); H = 16 causal 1024 11.6 / 14.3,
+// 2048 30.3 / 23.2 (staged); H = 4 causal 4096 29.8 / 35.2; H = 1 4096 26.8 / 34.6.
+bool fwd_short(int n_heads, int seq_len, bool causal) {
+  const long long nb = (seq_len + kShortRows - 1) / kShortRows, n64 = (seq_len + kBN - 1) / kBN;
+  const long long tiles = n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb);
+  return std::max(tiles * 200 / 256, nb * 620 / kShortWaves) < n64 * 566;
+}
+
 }  // namespace
 
 hipError_t launch_fwd_d64(const float *q, const float *k, const float *v, float *o, float *lse,
@@ -615,9 +833,18 @@ hipError_t launch_fwd_d64(const float *q, const float *k, const float *v, float 
   int qlo_stride = 0;
   if (bwd_workspace != nullptr)
     bwd_ws_qkv_copies(bwd_workspace, n_heads, seq_len, &q16, &k16, &v16, &qlo, &qlo_stride);
+  if (ldi <= 0) ldi = n_heads * kD;
+  if (fwd_short(n_heads, seq_len, causal)) {
+    const int n_blocks = (seq_len + kShortRows - 1) / kShortRows;
+    const int n_wg = n_blocks * n_heads;
+    hipLaunchKernelGGL(fwd_d64_short_kernel, dim3((unsigned)n_wg), dim3(64 * kShortWaves), 0, stream, q, k, v, o, lse,
+                       n_heads, seq_len, scale * kLog2e, causal ? 1 : 0, n_blocks, causal && n_wg <= 512 ? 1 : 0, q16,
+                       k16, v16, qlo, qlo_stride, ldi);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(fwd_d64_kernel, grid, dim3(kThreads), 0, stream, q, k, v, o, lse, n_heads,
                      seq_len, scale * kLog2e, causal ? 1 : 0, n_qtiles, q16, k16, v16, qlo, qlo_stride,
-                     ldi > 0 ? ldi : n_heads * kD);
+                     ldi);
   return hipGetLastError();
 }
 
