@@ -700,16 +700,10 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
   float m = -INFINITY, l = 0.f;
   f32x16 negm = f32x16{};  // -m in every register (0 while m = -inf)
   for (int t = wave; t < n_tiles; t += kShortWaves) {
-    const bool own = save && t == blk;  // the tile of the workgroup's own rows
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const half4_t kx = to_half4(kr[i]), vx = to_half4(vr[i]);
-      *reinterpret_cast<half4_t *>(kt + soff[i]) = kx;
-      *reinterpret_cast<half4_t *>(vt + soff[i]) = vx;
-      if (own) {
-        save4(K16, 1, t, i, kx, kr[i], 1.f);
-        save4(V16, -1, t, i, vx, vr[i], 1.f);
-      }
+      *reinterpret_cast<half4_t *>(kt + soff[i]) = to_half4(kr[i]);
+      *reinterpret_cast<half4_t *>(vt + soff[i]) = to_half4(vr[i]);
     }
     load_tile(K, t + kShortWaves, kr);
     load_tile(V, t + kShortWaves, vr);
@@ -720,6 +714,7 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
     for (int ds = 1; ds < 4; ++ds) s = mfma32x32x16(kf[ds], qf[ds], s);
     const int k0 = t * kShortRows;
     if (k0 + kShortRows - 1 > (causal ? q0 : S - 1)) {
+      asm volatile("");  // a branch, not 16 selects in every tile
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (k0 + 8 * (r >> 2) + 4 * hh + (r & 3) > key_lim) s[r] = -INFINITY;
@@ -767,6 +762,18 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
       for (int db = 0; db < 2; ++db) o[db] = mfma32x32x16(tile_tr8(vt, ks, db, lane), pf[ks], o[db]);
   }
 
+  if (save) {
+    // K and V of the workgroup's own rows, eight of them per wave, read again:
+    // keeping their tile's values through the loop costs it registers.
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int i = 2 * wave + k, off = ((4 * i + lrow) * ldi + lcol) * 4;
+      const float4 x = load4(tile(K, blk), off), y = load4(tile(V, blk), off);
+      save4(K16, 1, blk, i, to_half4(x), x, 1.f);
+      save4(V16, -1, blk, i, to_half4(y), y, 1.f);
+    }
+  }
+
   // Merge: each wave writes (m, l, O) (over its own tiles); wave w finishes
   // registers 4w .. 4w+3 of both blocks, values 32*db + 8w + 4*hh + 0..3.
   const float lsum = pair_sum(l);
@@ -812,10 +819,10 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
 // 256 CUs, but at least 620 ns for each of a wave's tiles in turn; the staged
 // one: 566 ns for each 64-key tile of its longest workgroup (when all of them
 // run at once; longer otherwise, and then the short kernel has lost anyway).
-// Measured, short against staged, us: H = 12 causal S = 128 5.0 / 7.1, 512 7.4 /
-// 10.0, 1024 11.4 / 14.1, 1536 15.7 / 17.8, 2048 25.3 / 22.7 (staged); unmasked
-// 512 7.6 / 11.6, 1536 28.8 / 19.8 (staged); H = 16 causal 1024 11.6 / 14.3,
-// 2048 30.3 / 23.2 (staged); H = 4 causal 4096 29.8 / 35.2; H = 1 4096 26.8 / 34.6.
+// Measured, short against staged, us: H = 12 causal S = 128 4.8 / 7.1, 512 7.0 /
+// 10.0, 1024 10.3 / 14.1, 1536 15.2 / 17.8, 2048 25.3 / 22.7 (staged); unmasked
+// 512 7.2 / 11.6, 1536 28.8 / 19.8 (staged); H = 16 causal 1024 10.8 / 14.3, 2048
+// 30.3 / 23.2 (staged); H = 4 causal 4096 28.3 / 35.2; H = 1 4096 24.7 / 34.6.
 bool fwd_short(int n_heads, int seq_len, bool causal) {
   const long long nb = (seq_len + kShortRows - 1) / kShortRows, n64 = (seq_len + kBN - 1) / kBN;
   const long long tiles = n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb);
