@@ -932,6 +932,338 @@ __global__ __launch_bounds__(kThreads) void bwd_main_kernel(BwdArgs a, Sched sch
   }
 }
 
+// ---------------------------------------------------------- short sequences
+// The kernel above takes 128 keys or query rows a workgroup and up to S/64
+// steps of 0.87 us (0.62 for dQ): at S = 1024 its 192 workgroups leave CUs idle
+// and the longest takes 16 steps. Here an item is 32 keys (dK/dV) or 32 query
+// rows (dQ), and the four waves of its workgroup take the 32-row tiles w, w + 4,
+// ... of the other side on their own, each through LDS tiles of its own, and add
+// their results at the end. The same products on the same fp16 copies, row
+// statistics, scales and residues; only the order of the sums differs.
+// A tile (4 KB, contiguous) is fetched into registers while the previous one is
+// worked on, a kilobyte per load, and stored to LDS. (Row fragments straight
+// from memory touch 32 lines per load, and 8 waves' tiles overflow the L1 in
+// between: 25.5 against 18.9 us for the kernel above at H = 12, S = 1024.)
+constexpr int kShortWaves = 4;
+constexpr int kShortRows = 32;
+constexpr int kShortTile = kShortRows * kD;  // halves
+// Per wave two tiles and a tile's row statistics (8.25 KB); at the end its dK and
+// dV (or dQ) registers (16 KB).
+constexpr int kShortLdsBytes = kShortWaves * 4 * 16 * 64 * 4;
+
+// The 32 rows from row0 (uniform) of one head of an fp16 copy (p: its row 0)
+// into registers: lane l of load i holds bytes 1024*i + 16*l of the tile, row
+// 8*i + l/8. Rows past n_rows read as zeros.
+__device__ __forceinline__ void short_load(const half_t *p, int n_rows, int row0, int lane, half8_t (&x)[4]) {
+  const auto rs = buffer_rsrc(p + (size_t)min(row0, n_rows) * kD,
+                              (unsigned)uniform_clamp0<kShortRows>(n_rows - row0) * kD * 2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    x[i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, 1024 * i + 16 * lane, 0, 0));
+}
+__device__ __forceinline__ void short_store(half_t *tile, int lane, const half8_t (&x)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<half8_t *>(tile + tile_off(8 * i + (lane >> 3), 8 * (lane & 7))) = x[i];
+}
+// Row fragment ds: lane c + 32*hh holds row c, values 16*ds + 8*hh + 0..7.
+__device__ __forceinline__ half8_t short_frag(const half_t *tile, int lane, int ds) {
+  return *reinterpret_cast<const half8_t *>(tile + tile_off(lane & 31, 8 * (2 * ds + (lane >> 5))));
+}
+// fp16(x - fp16(x)) of the slots of an accumulator (see kLoRows).
+__device__ __forceinline__ half8_t slot_residue(const f32x16 &x, half8_t rounded, int j) {
+  half8_t lo;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) lo[i] = (half_t)(x[8 * j + i] - (float)rounded[i]);
+  return lo;
+}
+
+// dK and dV of keys [key0, key0 + 32) of one head.
+__device__ __forceinline__ void dkdv_short(const BwdArgs &a, int head, int key0, unsigned char *lds_raw) {
+  const int lane = threadIdx.x & 63, c = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = a.S, key = key0 + c;
+  const size_t head_row = (size_t)head * S;
+  const half_t *Q = a.Q16 + head_row * kD, *G = a.dO16 + head_row * kD;
+  half_t *qt = reinterpret_cast<half_t *>(lds_raw) + wave * 2 * kShortTile, *gt = qt + kShortTile;
+  const int n_tiles = (S + kShortRows - 1) / kShortRows, first = a.causal ? key0 / kShortRows : 0;
+
+  float *st = reinterpret_cast<float *>(lds_raw) + kShortWaves * kShortTile + wave * 2 * kShortRows;
+
+  half8_t kf[4], vf[4], qx[4], gx[4];
+  float stat;  // lane c + 32*hh: row c's -lse*log2(e) (hh 0) or -Delta*sigma_b (hh 1)
+  auto fetch = [&](int t) {
+    const int q0 = t * kShortRows;
+    short_load(Q, S, q0, lane, qx);
+    short_load(G, S, q0, lane, gx);
+    const float *p = (hh ? a.deltan : a.lse2n) + head_row;
+    stat = q0 + c < S ? p[q0 + c] : 0.f;
+  };
+  short_load(a.K16 + head_row * kD, S, key0, lane, kf);
+  short_load(a.V16 + head_row * kD, S, key0, lane, vf);
+  fetch(first + wave);
+  short_store(qt, lane, kf);
+  short_store(gt, lane, vf);
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds) {
+    kf[ds] = short_frag(qt, lane, ds);
+    vf[ds] = short_frag(gt, lane, ds);
+  }
+
+  // The smallest dO scale of the item's blocks, the accumulators' unit, and
+  // whether all have it (see dkdv_path).
+  const float *sg = a.sigma + (size_t)head * a.n_blocks;
+  const int first_qb = first * kShortRows / kPreRows;
+  float mn = sg[first_qb], mx = mn;
+  for (int b = first_qb + lane; b < a.n_blocks; b += 64) {
+    mn = fminf(mn, sg[b]);
+    mx = fmaxf(mx, sg[b]);
+  }
+  const bool sig_uniform = !__any(mn != mx) && !__any(mn != __shfl(mn, 0, 64));
+  const int sig_min = __builtin_amdgcn_readfirstlane(__float_as_int(wave_min(mn)));
+
+  f32x16 dk[2], dv[2];
+  dk[0] = dk[1] = dv[0] = dv[1] = f32x16{};
+  for (int t = first + wave; t < n_tiles; t += kShortWaves) {
+    const int q0 = t * kShortRows;
+    short_store(qt, lane, qx);
+    short_store(gt, lane, gx);
+    st[lane] = stat;
+    fetch(t + kShortWaves);
+    // S - lse2 and dP - Delta: register r is row 8*(r/4) + 4*hh + r%4.
+    f32x16 s, dp;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 nl = *reinterpret_cast<const f32x4 *>(st + 8 * g + 4 * hh);
+      const f32x4 nd = *reinterpret_cast<const f32x4 *>(st + kShortRows + 8 * g + 4 * hh);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[4 * g + i] = nl[i];
+        dp[4 * g + i] = nd[i];
+      }
+    }
+    if (!sig_uniform) {
+      const int sig_b = __builtin_amdgcn_readfirstlane(__float_as_int(sg[q0 / kPreRows]));
+      const float lr = (float)(((sig_min >> 23) & 0xff) - ((sig_b >> 23) & 0xff));
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] += lr;
+    }
+    half8_t qa[4], ga[4];
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      qa[ds] = short_frag(qt, lane, ds);
+      ga[ds] = short_frag(gt, lane, ds);
+    }
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      s = mfma32x32x16(qa[ds], kf[ds], s);
+      dp = mfma32x32x16(ga[ds], vf[ds], dp);
+    }
+    // The transposed reads start before the exponentials, which hide them.
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t gtr[2][2], qtr[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        gtr[j][db] = tile_tr8(gt, j, db, lane);
+        qtr[j][db] = tile_tr8(qt, j, db, lane);
+      }
+    if (a.causal && t == first) {
+      asm volatile("");  // a branch, not 16 selects in every tile
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (key > q0 + (r >> 2) * 8 + hh * 4 + (r & 3)) s[r] = -INFINITY;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = fast_exp2(s[r]);
+      dp[r] *= s[r];
+    }
+    // Rows 0-63 against keys 0-127 (causal): the residues' products too.
+    const bool lo_corr = a.causal && key0 < kKeysPerWg && q0 < kLoRows;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const half8_t pf = acc_to_slots(s, j), dsf = acc_to_slots(dp, j);
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        dv[db] = mfma32x32x16(pf, gtr[j][db], dv[db]);
+        dk[db] = mfma32x32x16(dsf, qtr[j][db], dk[db]);
+      }
+    }
+    if (lo_corr) {
+      const half_t *lo = a.lo16 + (size_t)head * kLoTiles * kLoRows * kD;
+      half8_t x[4];
+      short_load(lo, min(S, kLoRows), q0, lane, x);
+      short_store(gt, lane, x);
+      short_load(lo + kLoRows * kD, min(S, kLoRows), q0, lane, x);
+      short_store(qt, lane, x);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const half8_t pf = acc_to_slots(s, j), dsf = acc_to_slots(dp, j), dsl = slot_residue(dp, dsf, j);
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+          dv[db] = mfma32x32x16(pf, tile_tr8(gt, j, db, lane), dv[db]);
+          dk[db] = mfma32x32x16(dsf, tile_tr8(qt, j, db, lane), dk[db]);
+          dk[db] = mfma32x32x16(dsl, qtr[j][db], dk[db]);
+        }
+      }
+    }
+  }
+
+  // Wave w adds up block w of dk[0], dk[1], dv[0], dv[1] over the waves, in wave order.
+  __syncthreads();
+  f32x4 *part = reinterpret_cast<f32x4 *>(lds_raw);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x16 &x = b < 2 ? dk[b & 1] : dv[b & 1];
+      part[((wave * 4 + b) * 4 + g) * 64 + lane] = f32x4{x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]};
+    }
+  __syncthreads();
+  const float sigma = __int_as_float(sig_min);
+  const float out_scale = wave < 2 ? kLn2 / sigma : 1.f / sigma;
+  float *out = (wave < 2 ? a.dK : a.dV) + head * kD + 32 * (wave & 1) + c;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    f32x4 x = part[(wave * 4 + g) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < kShortWaves; ++w) x += part[((w * 4 + wave) * 4 + g) * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int kr = key0 + 8 * g + 4 * hh + i;
+      if (kr < S) out[(size_t)kr * a.ldg] = x[i] * out_scale;
+    }
+  }
+}
+
+// dQ of query rows [q0, q0 + 32) of one head.
+__device__ __forceinline__ void dq_short(const BwdArgs &a, int head, int q0, unsigned char *lds_raw) {
+  const int lane = threadIdx.x & 63, c = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = a.S, query = q0 + c;
+  const size_t head_row = (size_t)head * S;
+  const half_t *K = a.K16 + head_row * kD, *V = a.V16 + head_row * kD;
+  half_t *kt = reinterpret_cast<half_t *>(lds_raw) + wave * 2 * kShortTile, *vt = kt + kShortTile;
+  const int n_tiles = ((a.causal ? min(S, q0 + kShortRows) : S) + kShortRows - 1) / kShortRows;
+  const int key_lim = a.causal ? min(query, S - 1) : S - 1;
+
+  half8_t qf[4], gf[4], kx[4], vx[4];
+  short_load(a.Q16 + head_row * kD, S, q0, lane, qf);
+  short_load(a.dO16 + head_row * kD, S, q0, lane, gf);
+  short_load(K, S, wave * kShortRows, lane, kx);
+  short_load(V, S, wave * kShortRows, lane, vx);
+  short_store(kt, lane, qf);
+  short_store(vt, lane, gf);
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds) {
+    qf[ds] = short_frag(kt, lane, ds);
+    gf[ds] = short_frag(vt, lane, ds);
+  }
+  // (Rows past S: P = 0.)
+  const float l = query < S ? a.lse2n[head_row + query] : -INFINITY;
+  const float d = query < S ? a.deltan[head_row + query] : 0.f;
+  f32x16 negL, negD;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    negL[r] = l;
+    negD[r] = d;
+  }
+  f32x16 dq[2];
+  dq[0] = dq[1] = f32x16{};
+  for (int t = wave; t < n_tiles; t += kShortWaves) {
+    const int k0 = t * kShortRows;
+    short_store(kt, lane, kx);
+    short_store(vt, lane, vx);
+    short_load(K, S, k0 + kShortWaves * kShortRows, lane, kx);
+    short_load(V, S, k0 + kShortWaves * kShortRows, lane, vx);
+    f32x16 s = negL, dp = negD;
+    half8_t ka[4], va[4];
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      ka[ds] = short_frag(kt, lane, ds);
+      va[ds] = short_frag(vt, lane, ds);
+    }
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      s = mfma32x32x16(ka[ds], qf[ds], s);
+      dp = mfma32x32x16(va[ds], gf[ds], dp);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    half8_t ktr[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int db = 0; db < 2; ++db) ktr[j][db] = tile_tr8(kt, j, db, lane);
+    if (k0 + kShortRows - 1 > (a.causal ? min(q0, S - 1) : S - 1)) {
+      asm volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + (r >> 2) * 8 + hh * 4 + (r & 3) > key_lim) s[r] = -INFINITY;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dp[r] *= fast_exp2(s[r]);
+    // Keys 0-63 of rows 0-127 (causal): the residues' products too.
+    const bool lo_corr = a.causal && q0 < kQueriesPerWg && k0 < kLoRows;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const half8_t dsf = acc_to_slots(dp, j);
+#pragma unroll
+      for (int db = 0; db < 2; ++db) {
+        dq[db] = mfma32x32x16(ktr[j][db], dsf, dq[db]);
+      }
+    }
+    if (lo_corr) {
+      half8_t x[4];
+      short_load(a.lo16 + ((size_t)head * kLoTiles + 2) * kLoRows * kD, min(S, kLoRows), k0, lane, x);
+      short_store(kt, lane, x);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const half8_t dsf = acc_to_slots(dp, j), dsl = slot_residue(dp, dsf, j);
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+          dq[db] = mfma32x32x16(tile_tr8(kt, j, db, lane), dsf, dq[db]);
+          dq[db] = mfma32x32x16(ktr[j][db], dsl, dq[db]);
+        }
+      }
+    }
+  }
+
+  // Wave w adds up registers 4w .. 4w+3 of both blocks: values 32*db + 8w + 4*hh + 0..3.
+  __syncthreads();
+  f32x4 *part = reinterpret_cast<f32x4 *>(lds_raw);
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      part[((wave * 2 + db) * 4 + g) * 64 + lane] =
+          f32x4{dq[db][4 * g], dq[db][4 * g + 1], dq[db][4 * g + 2], dq[db][4 * g + 3]};
+  __syncthreads();
+  if (query >= S) return;
+  const float dq_scale = a.scale / a.sigma[(size_t)head * a.n_blocks + q0 / kPreRows];
+  float *row = a.dQ + (size_t)query * a.ldg + head * kD + 8 * wave + 4 * hh;
+#pragma unroll
+  for (int db = 0; db < 2; ++db) {
+    f32x4 x = part[(db * 4 + wave) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < kShortWaves; ++w) x += part[((w * 2 + db) * 4 + wave) * 64 + lane];
+    *reinterpret_cast<float4 *>(row + 32 * db) =
+        make_float4(x[0] * dq_scale, x[1] * dq_scale, x[2] * dq_scale, x[3] * dq_scale);
+  }
+}
+
+// One workgroup per item, longest first: for rank r the dK/dV item of key block
+// r and the dQ item of query block n-1-r, for every head.
+__global__ __launch_bounds__(64 * kShortWaves, 2) void bwd_main_short_kernel(BwdArgs a, int n_items) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kShortLdsBytes];
+  const int item = __builtin_amdgcn_readfirstlane(blockIdx.x / a.H), head = blockIdx.x - item * a.H;
+  if ((item & 1) == 0)
+    dkdv_short(a, head, (item >> 1) * kShortRows, lds_raw);
+  else
+    dq_short(a, head, (n_items - 1 - (item >> 1)) * kShortRows, lds_raw);
+}
+
 }  // namespace
 
 size_t bwd_workspace_bytes_d64(int n_heads, int seq_len) { return ws_layout(n_heads, seq_len).total; }
@@ -989,6 +1321,20 @@ void build_xcd_order(Sched &sched, int n_heads) {
   sched.use_wg = 1;
 }
 
+// Which main kernel: both times estimated from what they measured, in ns above
+// their common fixed 4 us. The short kernel: 215 ns of one CU a 32 x 32 tile
+// (counted once for dK/dV and once for dQ) over 256 CUs; the other: 870 ns for
+// each 64-row block of its longest workgroup (when all of them run at once).
+// Measured, short against the other, us: H = 12 causal S = 128 5.9 / 6.9, 512 9.1
+// / 12.1, 1024 16.0 / 18.4, 2048 39.8 / 33.7; unmasked 512 10.4 / 11.3, 1024
+// 25.3 / 18.3; H = 4 causal 2048 19.3 / 29.1, 4096 52.2 / 54.4; H = 1 4096 25.5 /
+// 50.7; H = 16 1024 20.3 / 19.8 (the other).
+static bool bwd_short(int n_heads, int seq_len, bool causal) {
+  const double nb = (seq_len + kShortRows - 1) / kShortRows, n64 = (seq_len + kQBlock - 1) / kQBlock;
+  const double tiles = 2.0 * n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb);
+  return tiles * 215 / 256 < n64 * 870;
+}
+
 hipError_t launch_bwd_main_d64(const float *lse, float *d_q, float *d_k, float *d_v, const void *workspace,
                                int n_heads, int seq_len, float scale, bool causal, hipStream_t stream,
                                int ldg) {
@@ -1012,6 +1358,12 @@ hipError_t launch_bwd_main_d64(const float *lse, float *d_q, float *d_k, float *
   a.n_blocks = pre_blocks(seq_len);
   a.scale = scale;
   a.ldg = ldg > 0 ? ldg : n_heads * kD;
+  if (bwd_short(n_heads, seq_len, causal)) {
+    const int n_items = (seq_len + kShortRows - 1) / kShortRows;
+    hipLaunchKernelGGL(bwd_main_short_kernel, dim3((unsigned)(2 * n_items * n_heads)), dim3(64 * kShortWaves), 0,
+                       stream, a, n_items);
+    return hipGetLastError();
+  }
   Sched sched;
   sched.n_qblocks = (seq_len + kQBlock - 1) / kQBlock;
   sched.n_qtiles = (seq_len + kQueriesPerWg - 1) / kQueriesPerWg;
