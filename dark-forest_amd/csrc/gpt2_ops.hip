@@ -17,9 +17,11 @@
 #include "dfattn_status.h"
 #include "dfgpt2.h"
 
+#include <algorithm>
 #include <climits>
 #include <initializer_list>
 #include <string>
+#include <type_traits>
 
 namespace dfattn {
 namespace {
@@ -53,15 +55,17 @@ __global__ __launch_bounds__(256) void ln_fwd_vec_kernel(const float *__restrict
   float4 v[V];
   float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    const int c = lane + 64 * i;
-    v[i] = c < nv ? xr[c] : splat4(0.f);
-    if (y != nullptr && c < nv) {
-      const float4 yv = yr[c];
-      v[i] = make_float4(v[i].x + yv.x, v[i].y + yv.y, v[i].z + yv.z, v[i].w + yv.w);
-    }
-    s += hsum4(v[i]);
+  for (int i = 0; i < V; ++i) v[i] = lane + 64 * i < nv ? xr[lane + 64 * i] : splat4(0.f);
+  if (y != nullptr) {
+    float4 w[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) w[i] = lane + 64 * i < nv ? yr[lane + 64 * i] : splat4(0.f);
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      v[i] = make_float4(v[i].x + w[i].x, v[i].y + w[i].y, v[i].z + w[i].z, v[i].w + w[i].w);
   }
+#pragma unroll
+  for (int i = 0; i < V; ++i) s += hsum4(v[i]);
   if (sum_out != nullptr) {
     float4 *sr = reinterpret_cast<float4 *>(sum_out + (size_t)row * features);
 #pragma unroll
@@ -215,9 +219,10 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_generic_kernel(const float *__r
 // plus each workgroup's partial column sums of grad_out * x_hat and grad_out
 // (the parameter gradients' terms) and, when `planes` is 3, of grad_x itself
 // (the bias gradient of the linear layer whose output gradient grad_x is):
-// per lane over its row, then the four rows added in wave order through LDS,
-// into partial[blockIdx.x][plane][features]. colsum_partials_kernel adds the
-// workgroups' partials in order. The rows are read once for all of it.
+// per lane over its wave's `rows_per_wave` rows in order, then the four waves
+// added in order through LDS, into partial[blockIdx.x][plane][features].
+// colsum_partials_kernel adds the workgroups' partials in order. The rows are
+// read once for all of it.
 template <int V>
 __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const float *__restrict__ dout, const float *__restrict__ x,
                                                            const float *__restrict__ gamma,
@@ -225,54 +230,61 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const float *__restri
                                                            const float *__restrict__ rstds,
                                                            const float *__restrict__ residual,
                                                            float *__restrict__ grad_x, float *__restrict__ partial,
-                                                           int planes, int batch, int features) {
+                                                           int planes, int batch, int features, int rows_per_wave) {
   __shared__ __attribute__((aligned(16))) float part[4][3][V * 256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * 4 + wave;
-  const bool ok = row < batch;
   const int nv = features >> 2;
-  const float mean = ok ? means[row] : 0.f, rstd = ok ? rstds[row] : 0.f;
-  const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)row * features);
-  const float4 *dr = reinterpret_cast<const float4 *>(dout + (size_t)row * features);
-  float4 xh[V], ds[V], dv[V];
-  float sds = 0.f, sdsx = 0.f;
+  const float f = (float)features;
+  float4 acc[3][V];
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    const int c = lane + 64 * i;
-    xh[i] = ds[i] = dv[i] = splat4(0.f);
-    if (ok && c < nv) {
-      const float4 xv = xr[c];
-      dv[i] = dr[c];
-      const float4 g = gamma ? reinterpret_cast<const float4 *>(gamma)[c] : splat4(1.f);
-      xh[i] = make_float4((xv.x - mean) * rstd, (xv.y - mean) * rstd, (xv.z - mean) * rstd, (xv.w - mean) * rstd);
-      ds[i] = make_float4(dv[i].x * g.x, dv[i].y * g.y, dv[i].z * g.z, dv[i].w * g.w);
-      sds += hsum4(ds[i]);
-      sdsx += (ds[i].x * xh[i].x + ds[i].y * xh[i].y) + (ds[i].z * xh[i].z + ds[i].w * xh[i].w);
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[p][i] = splat4(0.f);
+  auto add = [](float4 &a, float4 b) { a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+  for (int k = 0; k < rows_per_wave; ++k) {
+    const unsigned row = (blockIdx.x * rows_per_wave + k) * 4u + wave;
+    if (row >= (unsigned)batch) break;
+    const float mean = means[row], rstd = rstds[row];
+    const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)row * features);
+    const float4 *dr = reinterpret_cast<const float4 *>(dout + (size_t)row * features);
+    float4 xh[V], ds[V];
+    float sds = 0.f, sdsx = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int c = lane + 64 * i;
+      xh[i] = ds[i] = splat4(0.f);
+      if (c < nv) {
+        const float4 xv = xr[c], dv = dr[c];
+        const float4 g = gamma ? reinterpret_cast<const float4 *>(gamma)[c] : splat4(1.f);
+        xh[i] = make_float4((xv.x - mean) * rstd, (xv.y - mean) * rstd, (xv.z - mean) * rstd, (xv.w - mean) * rstd);
+        ds[i] = make_float4(dv.x * g.x, dv.y * g.y, dv.z * g.z, dv.w * g.w);
+        sds += hsum4(ds[i]);
+        sdsx += (ds[i].x * xh[i].x + ds[i].y * xh[i].y) + (ds[i].z * xh[i].z + ds[i].w * xh[i].w);
+        add(acc[0][i], make_float4(dv.x * xh[i].x, dv.y * xh[i].y, dv.z * xh[i].z, dv.w * xh[i].w));
+        add(acc[1][i], dv);
+      }
+    }
+    const float sum_ds = wave_sum(sds), sum_dsx = wave_sum(sdsx), kf = rstd / f;
+    float4 *gr = reinterpret_cast<float4 *>(grad_x + (size_t)row * features);
+    const float4 *rr = reinterpret_cast<const float4 *>(residual + (size_t)row * features);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int c = lane + 64 * i;
+      if (c < nv) {
+        float4 o = make_float4(kf * (f * ds[i].x - sum_ds - xh[i].x * sum_dsx), kf * (f * ds[i].y - sum_ds - xh[i].y * sum_dsx),
+                               kf * (f * ds[i].z - sum_ds - xh[i].z * sum_dsx), kf * (f * ds[i].w - sum_ds - xh[i].w * sum_dsx));
+        if (residual != nullptr) add(o, rr[c]);
+        gr[c] = o;
+        add(acc[2][i], o);
+      }
     }
   }
-  const float sum_ds = wave_sum(sds), sum_dsx = wave_sum(sdsx);
-  const float f = (float)features, k = rstd / f;
-  float4 *gr = reinterpret_cast<float4 *>(grad_x + (size_t)row * features);
-  const float4 *rr = reinterpret_cast<const float4 *>(residual + (size_t)row * features);
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = lane + 64 * i;
-    float4 o = splat4(0.f);
-    if (ok && c < nv) {
-      o = make_float4(k * (f * ds[i].x - sum_ds - xh[i].x * sum_dsx), k * (f * ds[i].y - sum_ds - xh[i].y * sum_dsx),
-                      k * (f * ds[i].z - sum_ds - xh[i].z * sum_dsx), k * (f * ds[i].w - sum_ds - xh[i].w * sum_dsx));
-      if (residual != nullptr) {
-        const float4 r = rr[c];
-        o = make_float4(o.x + r.x, o.y + r.y, o.z + r.z, o.w + r.w);
-      }
-      gr[c] = o;
-    }
-    if (c < nv) {
-      *reinterpret_cast<float4 *>(&part[wave][0][4 * c]) =
-          make_float4(dv[i].x * xh[i].x, dv[i].y * xh[i].y, dv[i].z * xh[i].z, dv[i].w * xh[i].w);
-      *reinterpret_cast<float4 *>(&part[wave][1][4 * c]) = dv[i];
-      *reinterpret_cast<float4 *>(&part[wave][2][4 * c]) = o;
-    }
+    if (c < nv)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<float4 *>(&part[wave][p][4 * c]) = acc[p][i];
   }
   __syncthreads();
   float *dst = partial + (size_t)blockIdx.x * planes * features;
@@ -329,6 +341,15 @@ __global__ __launch_bounds__(256) void colsum_partials_kernel(const float *__res
 // out += sums, else out = sums. cols % 4 == 0 and 16-byte aligned rows.
 constexpr int kColStrip = 16;
 constexpr int kRowSlots = 256;  // 16 waves x 16 rows per load
+constexpr int kColAhead = 16;
+// Two strips share each 128-byte line, so workgroups of one XCD (blockIdx % 8)
+// take them in pairs: on different XCDs both fetch the line (4096 x 3072: 17.1 ->
+// 10.6 us, 8192 x 8192: 78 -> 48 us).
+__device__ __forceinline__ int strip_of(int b, int n_strips) {
+  if (b >= n_strips / 16 * 16) return b;
+  const int i = b >> 3, x = b & 7;
+  return 2 * ((i >> 1) * 8 + x) + (i & 1);
+}
 template <bool LN>
 __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restrict__ g, const float *__restrict__ x,
                                                           const float *__restrict__ means,
@@ -343,11 +364,29 @@ __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restric
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int slot = 16 * w + (lane >> 2);
   const int c4 = lane & 3;
-  const int col = blockIdx.x * kColStrip + 4 * c4;
+  const int strip = strip_of(blockIdx.x, gridDim.x);
+  const int col = strip * kColStrip + 4 * c4;
   float4 a0 = splat4(0.f), a1 = splat4(0.f);
   if (col < cols) {
+    int r = slot;
+    if constexpr (!LN) {
+      // kColAhead rows' loads in flight per thread, then their sums in order.
+      for (; r + (kColAhead - 1) * kRowSlots < rows; r += kColAhead * kRowSlots) {
+        float4 v[kColAhead];
+#pragma unroll
+        for (int k = 0; k < kColAhead; ++k)
+          v[k] = *reinterpret_cast<const float4 *>(g + (size_t)(r + k * kRowSlots) * cols + col);
+#pragma unroll
+        for (int k = 0; k < kColAhead; ++k) {
+          a0.x += v[k].x;
+          a0.y += v[k].y;
+          a0.z += v[k].z;
+          a0.w += v[k].w;
+        }
+      }
+    }
 #pragma unroll 4
-    for (int r = slot; r < rows; r += kRowSlots) {
+    for (; r < rows; r += kRowSlots) {
       const float4 gv = *reinterpret_cast<const float4 *>(g + (size_t)r * cols + col);
       if constexpr (LN) {
         const float4 xv = *reinterpret_cast<const float4 *>(x + (size_t)r * cols + col);
@@ -382,7 +421,7 @@ __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restric
   __syncthreads();
   if (tid < kPlanes * kColStrip) {
     const int plane = tid / kColStrip, t = tid % kColStrip;
-    const int c = blockIdx.x * kColStrip + t;
+    const int c = strip * kColStrip + t;
     float *o = plane ? out1 : out0;
     if (c < cols && o != nullptr) {
       float s = 0.f;
@@ -654,24 +693,38 @@ void ln_forward(const float *x, const float *y, const float *gamma, const float 
 void ln_backward_dx(const float *dout, const float *x, const float *gamma, const float *means, const float *rstds,
                     const float *residual, float *grad_x, int b, int f, hipStream_t stream);
 
-// The register-resident row path: features % 4 == 0, at most 1024, 16-byte
-// aligned tensors.
+// The register-resident row path: features % 4 == 0, at most 2048 (8 float4 a
+// lane: with its column sums the backward then takes 200 of the 256 registers
+// of two waves per SIMD), 16-byte aligned tensors. Above 1024 features rows used
+// to take the generic path, three reads of the row: at 8192 x 2048 add+LayerNorm
+// took 76 us and its backward 133 us, now 42 and 97.
 bool ln_vec(uint32_t features, std::initializer_list<const void *> ptrs) {
-  if (features % 4 != 0 || features > 1024) return false;
+  if (features % 4 != 0 || features > 2048) return false;
   for (const void *p : ptrs)
     if (p != nullptr && !al(p, 16)) return false;
   return true;
 }
 
+// Calls fn(integral_constant V) for the float4 per lane that a row of f takes.
+template <class Fn>
+void with_ln_vectors(int f, Fn fn) {
+  switch ((f / 4 + 63) / 64) {
+    case 1: fn(std::integral_constant<int, 1>{}); break;
+    case 2: fn(std::integral_constant<int, 2>{}); break;
+    case 3: fn(std::integral_constant<int, 3>{}); break;
+    case 4: fn(std::integral_constant<int, 4>{}); break;
+    case 5:
+    case 6: fn(std::integral_constant<int, 6>{}); break;
+    default: fn(std::integral_constant<int, 8>{}); break;
+  }
+}
+
 void ln_forward(const float *x, const float *y, const float *gamma, const float *beta, float *sum_out, float *out,
                 float *means, float *rstds, int b, int f, hipStream_t stream) {
   if (ln_vec((uint32_t)f, {x, y, out, sum_out, gamma, beta})) {
-    switch ((f / 4 + 63) / 64) {
-      case 1: launch_ln_fwd_v<1>(x, y, gamma, beta, sum_out, out, means, rstds, b, f, stream); break;
-      case 2: launch_ln_fwd_v<2>(x, y, gamma, beta, sum_out, out, means, rstds, b, f, stream); break;
-      case 3: launch_ln_fwd_v<3>(x, y, gamma, beta, sum_out, out, means, rstds, b, f, stream); break;
-      default: launch_ln_fwd_v<4>(x, y, gamma, beta, sum_out, out, means, rstds, b, f, stream); break;
-    }
+    with_ln_vectors(f, [&](auto v) {
+      launch_ln_fwd_v<decltype(v)::value>(x, y, gamma, beta, sum_out, out, means, rstds, b, f, stream);
+    });
   } else {
     hipLaunchKernelGGL(ln_fwd_generic_kernel, dim3((b + 3) / 4), dim3(256), 0, stream, x, y, gamma, beta, sum_out, out,
                        means, rstds, b, f);
@@ -681,12 +734,9 @@ void ln_forward(const float *x, const float *y, const float *gamma, const float 
 void ln_backward_dx(const float *dout, const float *x, const float *gamma, const float *means, const float *rstds,
                     const float *residual, float *grad_x, int b, int f, hipStream_t stream) {
   if (ln_vec((uint32_t)f, {dout, x, gamma, residual, grad_x})) {
-    switch ((f / 4 + 63) / 64) {
-      case 1: launch_ln_dx_v<1>(dout, x, gamma, means, rstds, residual, grad_x, b, f, stream); break;
-      case 2: launch_ln_dx_v<2>(dout, x, gamma, means, rstds, residual, grad_x, b, f, stream); break;
-      case 3: launch_ln_dx_v<3>(dout, x, gamma, means, rstds, residual, grad_x, b, f, stream); break;
-      default: launch_ln_dx_v<4>(dout, x, gamma, means, rstds, residual, grad_x, b, f, stream); break;
-    }
+    with_ln_vectors(f, [&](auto v) {
+      launch_ln_dx_v<decltype(v)::value>(dout, x, gamma, means, rstds, residual, grad_x, b, f, stream);
+    });
   } else {
     hipLaunchKernelGGL(ln_bwd_dx_generic_kernel, dim3((b + 3) / 4), dim3(256), 0, stream, dout, x, gamma, means, rstds,
                        residual, grad_x, b, f);
@@ -775,14 +825,6 @@ extern "C" size_t dfgpt2_layernorm_backward_fused_workspace_bytes(uint32_t batch
   return (size_t)((batch + 3) / 4) * 3 * features * sizeof(float);
 }
 
-template <int V>
-void launch_ln_fused_v(const float *dout, const float *x, const float *gamma, const float *means, const float *rstds,
-                       const float *residual, float *grad_x, float *partial, int planes, int batch, int features,
-                       hipStream_t stream) {
-  hipLaunchKernelGGL(ln_bwd_fused_kernel<V>, dim3((batch + 3) / 4), dim3(256), 0, stream, dout, x, gamma, means,
-                     rstds, residual, grad_x, partial, planes, batch, features);
-}
-
 extern "C" int dfgpt2_layernorm_backward_fused(const float *grad_out, const float *x, const float *gamma,
                                                const float *means, const float *rstds, const float *residual,
                                                float *grad_x, float *grad_gamma, float *grad_beta, float *grad_bias,
@@ -796,8 +838,12 @@ extern "C" int dfgpt2_layernorm_backward_fused(const float *grad_out, const floa
     return st;
   const int b = (int)batch, f = (int)features;
   const bool sums = grad_gamma != nullptr || grad_beta != nullptr || grad_bias != nullptr;
-  if (!sums || !ln_vec(features, {grad_out, x, gamma, residual, grad_x})) {
-    // Any width and alignment: the separate launches, the same results contract.
+  const int planes = grad_bias != nullptr ? 3 : 2;
+  const size_t need = (size_t)((batch + 3) / 4) * planes * features * sizeof(float);
+  const bool room = workspace != nullptr && workspace_bytes >= need && al(workspace, 4);
+  if (!sums || !ln_vec(features, {grad_out, x, gamma, residual, grad_x}) || (features > 1024 && !room)) {
+    // Any width and alignment, and wide rows without a workspace: the separate
+    // launches, the same results contract.
     ln_backward_dx(grad_out, x, gamma, means, rstds, residual, grad_x, b, f, stream);
     if (int st = launched(fn); st != DFATTN_OK || !sums) return st;
     if (grad_gamma != nullptr || grad_beta != nullptr)
@@ -808,21 +854,21 @@ extern "C" int dfgpt2_layernorm_backward_fused(const float *grad_out, const floa
                            f % 4 == 0 && al(grad_x, 16), stream);
     return launched(fn);
   }
-  const int planes = grad_bias != nullptr ? 3 : 2;
-  const size_t need = (size_t)((batch + 3) / 4) * planes * features * sizeof(float);
-  if (workspace == nullptr || workspace_bytes < need || !al(workspace, 4))
+  if (!room)
     return record_error(DFATTN_ERR_WORKSPACE, std::string(fn) + ": workspace must be non-null, 4-byte aligned and hold " +
                                                   std::to_string(need) + " bytes");
   float *partial = static_cast<float *>(workspace);
-  switch ((f / 4 + 63) / 64) {
-    case 1: launch_ln_fused_v<1>(grad_out, x, gamma, means, rstds, residual, grad_x, partial, planes, b, f, stream); break;
-    case 2: launch_ln_fused_v<2>(grad_out, x, gamma, means, rstds, residual, grad_x, partial, planes, b, f, stream); break;
-    case 3: launch_ln_fused_v<3>(grad_out, x, gamma, means, rstds, residual, grad_x, partial, planes, b, f, stream); break;
-    default: launch_ln_fused_v<4>(grad_out, x, gamma, means, rstds, residual, grad_x, partial, planes, b, f, stream); break;
-  }
+  // More rows per wave mean fewer partial sums to write and add up, as long as
+  // 512 workgroups remain (two per CU).
+  const int rows_per_wave = std::max(1, std::min(8, b / (4 * 512)));
+  const int n_parts = (b + 4 * rows_per_wave - 1) / (4 * rows_per_wave);
+  with_ln_vectors(f, [&](auto v) {
+    hipLaunchKernelGGL(ln_bwd_fused_kernel<decltype(v)::value>, dim3(n_parts), dim3(256), 0, stream, grad_out, x, gamma,
+                       means, rstds, residual, grad_x, partial, planes, b, f, rows_per_wave);
+  });
   if (int st = launched(fn); st != DFATTN_OK) return st;
-  hipLaunchKernelGGL(colsum_partials_kernel, dim3((planes * f + 15) / 16), dim3(256), 0, stream, partial,
-                     (b + 3) / 4, planes, f, grad_gamma, grad_beta, grad_bias);
+  hipLaunchKernelGGL(colsum_partials_kernel, dim3((planes * f + 15) / 16), dim3(256), 0, stream, partial, n_parts,
+                     planes, f, grad_gamma, grad_beta, grad_bias);
   return launched(fn);
 }
 

@@ -1,0 +1,89 @@
+"""The GPT-2 step's row kernels where their variants meet: LayerNorm rows of up to 8 float4 a lane and
+just past them, several rows per wave in the fused backward, the bias gradient's row blocks, and the
+cross-entropy at the ends of its register variants, with rows that start at any 4-byte address.
+
+Against plain PyTorch in float64. Everything is fp32: sums over n terms of either sign carry a relative
+error of about sqrt(n) u (u = 6e-8) in 2-norm, at most 6e-6 for the 8200 rows here; single values are
+held to 1e-4 of the largest."""
+import pytest
+
+from dfattn import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def check(name, got, want, rel=6e-6):
+    got, want = got.detach(), want.detach()
+    got, want = got.double(), want.double()
+    err = float((got - want).norm() / want.norm().clamp_min(1e-30))
+    worst = float((got - want).abs().max() / want.abs().max().clamp_min(1e-30))
+    assert err <= rel and worst <= 1e-4, f"{name}: rel {err:.1e}, max {worst:.1e}"
+
+
+@pytest.mark.parametrize("rows,features", [(1, 1028), (5, 1536), (7, 1600), (2051, 2048), (4097, 768), (8200, 1024),
+                                           (9, 2052), (6, 1030)])
+@pytest.mark.parametrize("workspace", [True, False])
+def test_layer_norm_widths(device, rows, features, workspace):
+    """With and without a workspace: only rows of at most 1024 features need one."""
+    import torch
+
+    if not workspace and features <= 1024:
+        pytest.skip("needs its workspace")
+    print(f"[gpu-rows] LayerNorm {rows} x {features} workspace={workspace}", flush=True)
+    torch.manual_seed(rows + features)
+    x, y, dy, res = (torch.randn(rows, features, device=device) for _ in range(4))
+    gamma, beta = torch.randn(features, device=device), torch.randn(features, device=device)
+    total, out, dx = (torch.empty_like(x) for _ in range(3))
+    stats = torch.empty(2, rows, device=device)
+    dg, db, dbias = (torch.empty(features, device=device) for _ in range(3))
+    ops.add_layer_norm_forward_into(x, y, gamma, beta, total, out, stats)
+    ws = torch.empty(ops.layer_norm_backward_fused_workspace_bytes(rows, features) // 4 if workspace else 1, device=device)
+    ops.layer_norm_backward_fused_into(dy, total, gamma, stats, res, dx, dg, db, dbias, ws)
+    dg2, db2, dx2 = (torch.empty_like(t) for t in (dg, db, dx))
+    ops.layer_norm_backward_residual_into(dy, total, gamma, stats, res, dx2, dg2, db2)
+    t64, g64, b64 = ((x + y).double().requires_grad_(True), gamma.double().requires_grad_(True),
+                     beta.double().requires_grad_(True))
+    o64 = torch.nn.functional.layer_norm(t64, (features,), g64, b64, 1e-5)
+    gt, gg, gb = torch.autograd.grad(o64, (t64, g64, b64), dy.double())
+    want = gt + res.double()
+    check("sum", total, t64)
+    check("out", out, o64)
+    for name, got, w in (("dx", dx, want), ("dgamma", dg, gg), ("dbeta", db, gb), ("dbias", dbias, want.sum(0)),
+                         ("dx apart", dx2, want), ("dgamma apart", dg2, gg), ("dbeta apart", db2, gb)):
+        check(name, got, w)
+
+
+@pytest.mark.parametrize("rows", [1, 255, 4095, 4096, 4097, 8192])
+def test_bias_gradient_row_blocks(device, rows):
+    import torch
+
+    print(f"[gpu-rows] bias gradient rows={rows}", flush=True)
+    g = torch.randn(rows, 36, device=device)
+    check("bias", ops.bias_grad(g), g.double().sum(0))
+
+
+@pytest.mark.parametrize("cols", [1, 3, 2047, 2048, 2049, 8192, 8195, 16384, 16385, 30720, 30721, 50257, 51200, 51201])
+def test_cross_entropy_lengths(device, cols):
+    """One row all -1e30 but its target, and one whose largest logit comes last."""
+    import torch
+
+    print(f"[gpu-rows] cross-entropy cols={cols}", flush=True)
+    torch.manual_seed(cols)
+    rows = 5
+    logits = torch.randn(rows, cols, device=device) * 3
+    targets = torch.randint(0, cols, (rows,), device=device)
+    logits[1] = -1e30
+    logits[1, targets[1]] = 2.0
+    logits[2, cols - 1] = 60.0
+    want = torch.softmax(logits.double(), 1)
+    row_loss = -torch.log(want[torch.arange(rows), targets].clamp_min(1e-12)) / 7
+    want[torch.arange(rows), targets] -= 1
+    guard = torch.full((rows * cols + 8,), 7.0, device=device)
+    grad = guard[4:4 + rows * cols].view(rows, cols)
+    loss = torch.empty(rows, device=device)
+    ops.logit_ce_chunk(logits, targets.int(), grad, loss, 7)
+    check("grad", grad, want / 7)
+    check("loss", loss, row_loss)
+    assert (guard[:4] == 7).all() and (guard[4 + rows * cols:] == 7).all()
+    ops.logit_ce_chunk(logits, targets.int(), logits, loss, 7)  # in place
+    assert torch.equal(logits, grad)
