@@ -32,6 +32,7 @@ scaled_dot_product_attention and torch's AdamW, differentiated by autograd.
 """
 from __future__ import annotations
 
+import gc
 import math
 import os
 import struct
@@ -249,6 +250,10 @@ class StaticGPT2:
             for _ in range(warmup):
                 self.step(self._tokens, self._targets)
         torch.cuda.current_stream().wait_stream(side)
+        # A model that went out of use waits for the cycle collector (its engine refers to it), and
+        # its recorded graph waits for the device when it is freed, which ends the process if that
+        # happens inside a recording: so such models go now.
+        gc.collect()
         self._graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self._graph):
             self._loss = self.step(self._tokens, self._targets)

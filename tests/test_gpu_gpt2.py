@@ -126,6 +126,38 @@ def test_captured_step_replays_match_eager_steps(device):
         assert torch.allclose(a, b, rtol=0, atol=1e-6)
 
 
+def test_capture_frees_models_out_of_use_before_recording(device):
+    """A captured model that went out of use is freed before another one's recording starts: the cycle
+    collector, run inside the recording, finds none (freeing a recorded graph there ends the process)."""
+    import gc
+    import weakref
+
+    import torch
+
+    cfg = dict(vocab_size=500, d_model=64, n_heads=2, n_layers=1, d_ff=256, seq_len=64, seed=5)
+    tokens, targets = synthetic_batch(500, 64, 19, device)
+    gc.disable()
+    try:
+        old = StaticGPT2(**cfg, capturable=True)
+        old.capture(tokens, targets)
+        old.replay()
+        torch.cuda.synchronize()
+        left = weakref.ref(old)
+        del old
+        new = StaticGPT2(**cfg, capturable=True)
+        alive = []
+        backward = new._engine._backward
+        new._engine._backward = lambda: (alive.append(left() is not None), backward())
+        loss = new.capture(tokens, targets, warmup=0)
+        say(f"old model alive while recording: {alive}")
+        assert alive == [False]
+        new.replay()
+        torch.cuda.synchronize()
+        assert math.isfinite(float(loss))
+    finally:
+        gc.enable()
+
+
 def test_replay_after_checkpoint_load_records_the_step_again(device, tmp_path):
     """load_checkpoint drops the recorded step; the next replay records it again (the engine
     re-captures on its next step, static_gpt2.rs:619-629, 2111) and trains from the loaded state:
