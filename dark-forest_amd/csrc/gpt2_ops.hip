@@ -16,6 +16,7 @@
 #include "dfattn_internal.h"
 #include "dfattn_status.h"
 #include "dfgpt2.h"
+#include "gpt2_device.h"
 
 #include <algorithm>
 #include <climits>
@@ -27,9 +28,6 @@ namespace dfattn {
 namespace {
 
 constexpr float kLnEps = 1e-5f;  // layernorm.cu:14
-// tanh GELU constants: sqrt(2/pi) and the cubic coefficient (elementwise.cu:181-182).
-constexpr float kGeluK0 = 0.7978845608028654f;
-constexpr float kGeluK1 = 0.044715f;
 
 __device__ __forceinline__ float4 splat4(float a) { return make_float4(a, a, a, a); }
 __device__ __forceinline__ float hsum4(float4 v) { return (v.x + v.y) + (v.z + v.w); }
@@ -457,15 +455,6 @@ __global__ __launch_bounds__(256) void colsum_generic_kernel(const float *__rest
 }
 
 // ------------------------------------------------------------------- GELU
-__device__ __forceinline__ float gelu_f(float v) {
-  return 0.5f * v * (1.f + tanhf(kGeluK0 * (v + kGeluK1 * v * v * v)));
-}
-__device__ __forceinline__ float gelu_grad(float go, float v) {
-  const float t = tanhf(kGeluK0 * (v + kGeluK1 * v * v * v));
-  const float d_inner = kGeluK0 * (1.f + 3.f * kGeluK1 * v * v);
-  return go * (0.5f * (1.f + t) + 0.5f * v * (1.f - t * t) * d_inner);
-}
-
 // out = gelu(x) (BWD: out = go * gelu'(x)); grid-stride over float4 groups
 // when every pointer is 16-byte aligned, the n % 4 tail by the first threads.
 template <bool BWD>

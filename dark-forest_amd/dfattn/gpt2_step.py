@@ -22,10 +22,12 @@ Mirrors the reference's static engine (darkforest-core/src/engine/static_gpt2.rs
 On the GPU (attention="dfattn") the step is the engine's own explicit forward and backward, with no
 autograd: every activation and backward scratch buffer is a view of one allocation sized at
 construction (`_NativeEngine`), the weights, gradients and AdamW moments are one more
-(`ops.ParamArena`), and every kernel but the GEMMs is this library's (include/dfgpt2.h and the
+(`ops.ParamArena`), and every kernel but part of the GEMMs is this library's (include/dfgpt2.h and the
 attention contexts): embedding gather and gradient, LayerNorm, tanh GELU, the bias gradients, the
-chunked fused cross-entropy and one AdamW launch over the whole arena, all fp32; the GEMMs are
-hipBLASLt / rocBLAS fp32, with per-shape solutions TunableOp measured (GEMM_SOLUTIONS).
+chunked fused cross-entropy and one AdamW launch over the whole arena, all fp32. The linear layers'
+fast products are dfgpt2_linear_* at the sizes where those are faster (`_own_gemms`); lm_head's, the
+exact ones and all at larger sizes are hipBLASLt / rocBLAS fp32, with per-shape solutions TunableOp
+measured (GEMM_SOLUTIONS).
 attention="sdpa", and any model on the CPU, is the reference's own parity comparator
 instead (scripts/verify_loss_parity.py:58): the same model in plain PyTorch operators with torch's
 scaled_dot_product_attention and torch's AdamW, differentiated by autograd.
@@ -159,8 +161,8 @@ class StaticGPT2:
         # run continue bit for bit.
         hp = dict(lr=_f32(lr), betas=(_f32(0.9), _f32(0.95)), eps=_f32(1e-8), weight_decay=_f32(0.1))
         self.native = self.device.type == "cuda" and attention == "dfattn"
-        # The engine's GEMMs take hipBLASLt's fast fp32 path (torch's allow_tf32 on ROCm): relative
-        # error ~5e-6 on these shapes against 1e-6 for the exact path, far inside the TF32 the
+        # The engine's GEMMs take the fast fp32 path (dfgpt2_linear_*, or hipBLASLt's by torch's
+        # allow_tf32 on ROCm): relative error ~5e-6 on these shapes against 1e-6 for the exact path, far inside the TF32 the
         # reference's cuBLAS GEMMs use (lib.rs:45-48), and up to 2.3x faster on the lm_head GEMM.
         self.fast_gemm = fast_gemm
         # tuned_gemms: the engine's GEMMs take the solutions in GEMM_SOLUTIONS (TunableOp, no tuning
@@ -355,8 +357,8 @@ class _NativeEngine:
         self.ids, self.tgt, self.pos = ints[:S], ints[w:w + S], ints[2 * w:2 * w + S]
         self.pos.copy_(torch.arange(S, dtype=torch.int32, device=dev))
         self.ctx = [AttentionContext(H, S, d // H, reuse_forward=True) for _ in range(L)]
-        # In a captured step the backward's weight-gradient GEMMs run on this stream, beside the
-        # input-gradient ones (eager dispatch of the cross-stream waits costs more than it gains).
+        # In a captured step hipBLASLt's weight-gradient GEMMs run on this stream, beside the
+        # input-gradient ones, where all of the step's are hipBLASLt's (eager dispatch of the cross-stream waits costs more than it gains).
         self.side = torch.cuda.Stream(device=dev) if torch.device(dev).type == "cuda" else None
         self._overlap = False
         self.scale = (d / H) ** -0.5
@@ -389,8 +391,8 @@ class _NativeEngine:
         return w
 
     # Per GEMM call site: the exact fp32 path (True) or the fast one, whichever measured faster at
-    # that site with the tuned solutions (whole replayed steps: qkv_fwd exact is 0.12 ms slower,
-    # qkv_dw and wo_dx exact no faster). *_fwd: the forward product (o and fc2 with the bias in the
+    # that site with the library's tuned solutions (whole replayed steps: qkv_fwd exact is 0.12 ms
+    # slower, qkv_dw and wo_dx exact no faster). *_fwd: the forward product (o and fc2 with the bias in the
     # GEMM's epilogue); *_dx / *_dw: the input and weight gradients.
     EXACT_SITES = {"qkv_fwd": False, "o_fwd": True, "fc1_fwd": False, "fc2_fwd": True,
                    "fc2_dx": False, "fc2_dw": False, "fc1_dx": True, "fc1_dw": False,
@@ -405,23 +407,44 @@ class _NativeEngine:
         torch = _torch()
         torch.backends.cuda.matmul.allow_tf32 = (not flag) and _NativeEngine._fast
 
-    def _linear(self, x, w, b, out, exact=True):
-        """out = x W^T + b (static_gpt2.rs linear_into; hipBLASLt). exact: one GEMM with the bias in
-        its epilogue on the exact fp32 path; otherwise the fast-path GEMM, then the bias added in
-        place (dfgpt2_add_bias)."""
+    def _own_gemms(self):
+        """Whether the step's fast sites run on dfgpt2_linear_* (the fast path's accuracy) rather than
+        on hipBLASLt: while the largest of their products is at most one 128 x 96 tile per CU. Up to
+        there they measured faster at every size and site (us in a graph, hipBLASLt first, GPT-2
+        small's widths: fc1_fwd 25.2 and 24.9 with its bias and GELU still to come for hipBLASLt,
+        qkv_fwd 25.0 and 23.7, qkv_dw 29.7 and 21.0, wo_dx 15.2 and 10.3; at 64 rows 11.1 and 9.9);
+        past it the library's larger tiles win (2048 rows: qkv_fwd 37 and 48). All of a step or
+        none, because these kernels fill a CU's LDS and gain nothing from a second stream: the whole
+        step takes 6.51 ms on one stream, 6.99 on two; on hipBLASLt 6.99 and 6.74."""
+        S, d, F = self.m.seq_len, self.m.d_model, self.m.d_ff
+        products = ((S, 3 * d), (S, F), (d, F), (F, d), (3 * d, d), (S, d))
+        return self.m.fast_gemm and max(-(-r // 128) * -(-c // 96) for r, c in products) <= 256
+
+    def _linear(self, x, w, b, out, exact=True, gelu_out=None):
+        """out = x W^T + b (static_gpt2.rs linear_into), and gelu_out = gelu(out) unless None. exact:
+        one hipBLASLt GEMM with the bias in its epilogue on the exact fp32 path; otherwise one
+        dfgpt2_linear_forward, or the fast-path GEMM and then the bias added in place, by GELU's
+        kernel where there is one."""
         torch = _torch()
-        if exact:
-            self._exact(True)
+        if not exact and self._own_gemms():
+            _ops.linear_forward_into(x, w, b, out, gelu_out)
+            return
+        self._exact(exact)
+        if exact and gelu_out is None:
             torch.addmm(b, x, w.t(), out=out)
-            self._exact(False)
         else:
             torch.mm(x, w.t(), out=out)
-            _ops.add_bias_into(out, b)
+            if gelu_out is None:
+                _ops.add_bias_into(out, b)
+            else:
+                _ops.bias_gelu_forward_into(out, b, gelu_out)
+        self._exact(False)
 
-    def _linear_backward(self, x, w, dy, dx, exact_dx=False, exact_dw=False, bias=None):
+    def _linear_backward(self, x, w, dy, dx, exact_dx=False, exact_dw=False, bias=None, gelu_in=None):
         """dx = dy W and W's gradient dy^T x, into the arena gradient view (static_gpt2.rs
         linear_backward_into); exact_dx / exact_dw: that product on the exact fp32 GEMM path;
-        bias: its gradient too (the column sums of dy), beside W's."""
+        bias: its gradient too (the column sums of dy), beside W's; gelu_in: x is gelu(gelu_in) and
+        dx becomes gelu_in's gradient."""
         torch = _torch()
         if self._overlap:
             # The previous weight gradient has finished before this one starts (and before the main
@@ -429,19 +452,30 @@ class _NativeEngine:
             main = torch.cuda.current_stream()
             main.wait_stream(self.side)
             self.side.wait_stream(main)
-        self._exact(exact_dx)
-        torch.mm(dy, w, out=dx)
-        self._exact(exact_dw)
+        if not exact_dx and self._own_gemms():
+            _ops.linear_backward_input_into(dy, w, dx, gelu_in)
+        else:
+            self._exact(exact_dx)
+            product = dx if gelu_in is None else self.b["da"]
+            torch.mm(dy, w, out=product)
+            if gelu_in is not None:
+                _ops._check(_ops.ops_lib().dfgpt2_gelu_backward(
+                    _ops._dev_ptr(product), _ops._dev_ptr(gelu_in), _ops._dev_ptr(dx), dx.numel(), _ops._stream_ptr()))
         if self._overlap:
             with torch.cuda.stream(self.side):
-                torch.mm(dy.t(), x, out=w.grad)
-                if bias is not None:
-                    self._bias_grad(dy, bias)
+                self._weight_grad(x, w, dy, exact_dw, bias)
         else:
-            torch.mm(dy.t(), x, out=w.grad)
-            if bias is not None:
-                self._bias_grad(dy, bias)
+            self._weight_grad(x, w, dy, exact_dw, bias)
         self._exact(False)
+
+    def _weight_grad(self, x, w, dy, exact, bias):
+        if not exact and self._own_gemms():
+            _ops.linear_backward_weight_into(dy, x, w.grad)
+        else:
+            self._exact(exact)
+            _torch().mm(dy.t(), x, out=w.grad)
+        if bias is not None:
+            self._bias_grad(dy, bias)
 
     @staticmethod
     def _bias_grad(dy, b):
@@ -472,8 +506,8 @@ class _NativeEngine:
     # ---------------------------------------------------------------- forward (static_gpt2.rs:1286-1373)
     def _forward(self):
         """Each residual add runs inside the LayerNorm that follows it (x_mid and LayerNorm 2, then
-        x_in[l+1] and the next layer's LayerNorm 1 or the final one), and the first MLP bias inside
-        GELU; the values are those of the separate operations."""
+        x_in[l+1] and the next layer's LayerNorm 1 or the final one), and the first MLP bias and
+        GELU inside the product or one kernel after it; the values are those of the separate operations."""
         torch = _torch()
         m, b, ex = self.m, self.b, self.exact_sites
         S, L = m.seq_len, m.n_layers
@@ -492,11 +526,7 @@ class _NativeEngine:
             self.ctx[l].forward_device_into(*self._qkv(l), self.scale, True, att)
             self._linear(att, lw["wo"], lw["bo"], b["tmp"], ex["o_fwd"])
             _ops.add_layer_norm_forward_into(x, b["tmp"], lw["ln2_g"], lw["ln2_b"], xmid, ln2, b[f"st2{l}"])
-            # h = ln2 W1^T; the bias goes into h as GELU reads it
-            self._exact(ex["fc1_fwd"])
-            torch.mm(ln2, lw["w1"].t(), out=b[f"h{l}"])
-            self._exact(False)
-            _ops.bias_gelu_forward_into(b[f"h{l}"], lw["b1"], b[f"a{l}"])
+            self._linear(ln2, lw["w1"], lw["b1"], b[f"h{l}"], ex["fc1_fwd"], gelu_out=b[f"a{l}"])
             self._linear(b[f"a{l}"], lw["w2"], lw["b2"], b["tmp"], ex["fc2_fwd"])
             if l + 1 < L:
                 nxt = m.layers[l + 1]
@@ -545,7 +575,8 @@ class _NativeEngine:
     # ---------------------------------------------------------------- backward (static_gpt2.rs:1424-1575)
     def _backward(self):
         m, b, ex = self.m, self.b, self.exact_sites
-        self._overlap = self.side is not None and _torch().cuda.is_current_stream_capturing()
+        self._overlap = (self.side is not None and not self._own_gemms()
+                         and _torch().cuda.is_current_stream_capturing())
         if self._overlap:
             self.side.wait_stream(_torch().cuda.current_stream())
         L = m.n_layers
@@ -557,10 +588,7 @@ class _NativeEngine:
         for l in reversed(range(L)):
             lw = m.layers[l]
             # MLP: g is d(x_in[l+1]) = d(mlp out) = d(x_mid) through the residual
-            self._linear_backward(b[f"a{l}"], lw["w2"], g, b["da"], ex["fc2_dx"], ex["fc2_dw"])
-            _ops._check(_ops.ops_lib().dfgpt2_gelu_backward(_ops._dev_ptr(b["da"]), _ops._dev_ptr(b[f"h{l}"]),
-                                                            _ops._dev_ptr(b["dh"]), b["dh"].numel(),
-                                                            _ops._stream_ptr()))
+            self._linear_backward(b[f"a{l}"], lw["w2"], g, b["dh"], ex["fc2_dx"], ex["fc2_dw"], gelu_in=b[f"h{l}"])
             self._linear_backward(b[f"ln2{l}"], lw["w1"], b["dh"], b["dln"], ex["fc1_dx"], ex["fc1_dw"], lw["b1"])
             # d(x_mid) = g + LayerNorm 2's gradient
             self._ln_backward(b["dln"], b[f"xmid{l}"], lw["ln2_g"], lw["ln2_b"], b[f"st2{l}"], other, residual=g,

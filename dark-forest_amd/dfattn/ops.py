@@ -54,6 +54,9 @@ SYMBOLS = {
     "launch_add": (None, [_P] * 3 + [_U32]),
     "launch_scale": (None, [_P, _F, _P, _U32]),
     "dfgpt2_add_bias": (_I, [_P] * 3 + [_U32, _U32, _P]),
+    "dfgpt2_linear_forward": (_I, [_P] * 5 + [_U32, _U32, _U32, _P]),
+    "dfgpt2_linear_backward_input": (_I, [_P] * 4 + [_U32, _U32, _U32, _P]),
+    "dfgpt2_linear_backward_weight": (_I, [_P] * 3 + [_U32, _U32, _U32, _P]),
     "dfgpt2_layernorm_backward_fused": (_I, [_P] * 11 + [_SZ, _U32, _U32, _P]),
 }
 
@@ -150,6 +153,27 @@ def bias_gelu_forward_into(h, bias, out):
     """dfgpt2_bias_gelu_forward: h += bias (per column, in place), out = gelu(h)."""
     rows, cols = _rows_cols(h)
     _check(ops_lib().dfgpt2_bias_gelu_forward(_dev_ptr(h), _dev_ptr(bias), _dev_ptr(out), rows, cols, _stream_ptr()))
+
+
+def linear_forward_into(x, w, bias, out, gelu_out=None):
+    """dfgpt2_linear_forward: out = x w^T + bias, and gelu_out = gelu(out) unless None."""
+    (rows, k), n = _rows_cols(x), w.shape[0]
+    _check(ops_lib().dfgpt2_linear_forward(_dev_ptr(x), _dev_ptr(w), _dev_ptr(bias), _dev_ptr(out), _dev_ptr(gelu_out),
+                                           rows, k, n, _stream_ptr()))
+
+
+def linear_backward_input_into(grad_out, w, grad_x, gelu_in=None):
+    """dfgpt2_linear_backward_input: grad_x = grad_out w, times gelu'(gelu_in) unless None."""
+    (rows, n), k = _rows_cols(grad_out), w.shape[1]
+    _check(ops_lib().dfgpt2_linear_backward_input(_dev_ptr(grad_out), _dev_ptr(w), _dev_ptr(gelu_in), _dev_ptr(grad_x),
+                                                  rows, k, n, _stream_ptr()))
+
+
+def linear_backward_weight_into(grad_out, x, grad_w):
+    """dfgpt2_linear_backward_weight: grad_w = grad_out^T x."""
+    (rows, n), k = _rows_cols(grad_out), x.shape[1]
+    _check(ops_lib().dfgpt2_linear_backward_weight(_dev_ptr(grad_out), _dev_ptr(x), _dev_ptr(grad_w), rows, k, n,
+                                                   _stream_ptr()))
 
 
 def bias_grad(grad_out):

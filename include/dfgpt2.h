@@ -139,6 +139,22 @@ int dfgpt2_layernorm_backward_fused(const float *grad_out, const float *x, const
  * out must not overlap h.                                                                      */
 int dfgpt2_bias_gelu_forward(float *h, const float *bias, float *out, uint32_t rows, uint32_t cols,
                              hipStream_t stream);
+/* A linear layer's products on the bf16 matrix cores from fp32 operands (each value as the sum of
+ * two bf16 terms, three products summed in fp32: about 4.4e-6 relative to the exact product's
+ * norm; the reference's are TF32, lib.rs:45-48). Row-major tensors without padding, w
+ * [out_features, in_features]; outputs must not overlap inputs. Results are reproducible bit for bit. A finite value that rounds
+ * to infinity in bf16 (above 3.39e38), and an infinity, give NaN.
+ * forward (linear_into, then gelu, static_gpt2.rs:1353-1355): out = x w^T + bias, and gelu_out =
+ * gelu(out) unless NULL; [rows, out_features].
+ * backward_input: grad_x = grad_out w, [rows, in_features]; with gelu_in (not NULL), times gelu'(gelu_in):
+ * dfgpt2_gelu_backward of the product.
+ * backward_weight: grad_w = grad_out^T x, overwritten (zeros when rows == 0).                  */
+int dfgpt2_linear_forward(const float *x, const float *w, const float *bias, float *out, float *gelu_out,
+                          uint32_t rows, uint32_t in_features, uint32_t out_features, hipStream_t stream);
+int dfgpt2_linear_backward_input(const float *grad_out, const float *w, const float *gelu_in, float *grad_x,
+                                 uint32_t rows, uint32_t in_features, uint32_t out_features, hipStream_t stream);
+int dfgpt2_linear_backward_weight(const float *grad_out, const float *x, float *grad_w, uint32_t rows,
+                                  uint32_t in_features, uint32_t out_features, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -72,4 +72,12 @@ extern "C" {
                                            stream: *mut c_void) -> c_int;
     pub fn dfgpt2_bias_gelu_forward(h: *mut f32, bias: *const f32, out: *mut f32, rows: u32, cols: u32,
                                     stream: *mut c_void) -> c_int;
+    pub fn dfgpt2_linear_forward(x: *const f32, w: *const f32, bias: *const f32, out: *mut f32,
+                                 gelu_out: *mut f32, rows: u32, in_features: u32, out_features: u32,
+                                 stream: *mut c_void) -> c_int;
+    pub fn dfgpt2_linear_backward_input(grad_out: *const f32, w: *const f32, gelu_in: *const f32,
+                                        grad_x: *mut f32, rows: u32, in_features: u32, out_features: u32,
+                                        stream: *mut c_void) -> c_int;
+    pub fn dfgpt2_linear_backward_weight(grad_out: *const f32, x: *const f32, grad_w: *mut f32, rows: u32,
+                                         in_features: u32, out_features: u32, stream: *mut c_void) -> c_int;
 }
