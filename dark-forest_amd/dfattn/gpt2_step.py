@@ -39,6 +39,7 @@ import math
 import os
 import struct
 import time
+import weakref
 
 from . import AttentionContext
 from . import ops as _ops
@@ -252,13 +253,18 @@ class StaticGPT2:
             for _ in range(warmup):
                 self.step(self._tokens, self._targets)
         torch.cuda.current_stream().wait_stream(side)
-        # A model that went out of use waits for the cycle collector (its engine refers to it), and
-        # its recorded graph waits for the device when it is freed, which ends the process if that
-        # happens inside a recording: so such models go now.
-        gc.collect()
-        self._graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self._graph):
-            self._loss = self.step(self._tokens, self._targets)
+        # Freeing a recorded graph waits for the device, which ends the process if it happens inside a
+        # recording. A model out of use is freed at once (its engine holds no reference to it), and one
+        # that a caller's own cycle keeps is left to a collection after the recording.
+        collecting = gc.isenabled()
+        gc.disable()
+        try:
+            self._graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(self._graph):
+                self._loss = self.step(self._tokens, self._targets)
+        finally:
+            if collecting:
+                gc.enable()
         return self._loss
 
     def set_batch(self, tokens, targets):
@@ -298,7 +304,7 @@ class _NativeEngine:
 
     def __init__(self, m: StaticGPT2):
         torch = _torch()
-        self.m = m
+        self.m = weakref.proxy(m)  # no cycle: a model's memory and graph go with its last reference
         self.exact_sites = dict(self.EXACT_SITES)
         S, d, F, V, L, H = m.seq_len, m.d_model, m.d_ff, m.vocab_size, m.n_layers, m.n_heads
         self.chunk = min(S, 512)  # static_gpt2.rs:423

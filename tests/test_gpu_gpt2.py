@@ -158,6 +158,36 @@ def test_capture_frees_models_out_of_use_before_recording(device):
         gc.enable()
 
 
+def test_no_cycle_collection_inside_a_recording(device):
+    """A captured model held by a caller's own cycle is not collected inside another one's recording, and
+    the collector is as it was afterwards."""
+    import gc
+    import weakref
+
+    import torch
+
+    cfg = dict(vocab_size=500, d_model=64, n_heads=2, n_layers=1, d_ff=256, seq_len=64, seed=5)
+    tokens, targets = synthetic_batch(500, 64, 19, device)
+    old = StaticGPT2(**cfg, capturable=True)
+    old.capture(tokens, targets)
+    torch.cuda.synchronize()
+    left, cycle = weakref.ref(old), [old]
+    cycle.append(cycle)
+    new = StaticGPT2(**cfg, capturable=True)
+    seen = []
+    backward = new._engine._backward
+    new._engine._backward = lambda: (seen.append(gc.isenabled()), backward())
+    assert gc.isenabled()
+    del old, cycle
+    new.capture(tokens, targets, warmup=0)
+    say(f"collector on while recording: {seen}")
+    assert seen == [False] and gc.isenabled()
+    del new._engine._backward  # the lambda's own cycle
+    torch.cuda.synchronize()
+    gc.collect()
+    assert left() is None
+
+
 def test_replay_after_checkpoint_load_records_the_step_again(device, tmp_path):
     """load_checkpoint drops the recorded step; the next replay records it again (the engine
     re-captures on its next step, static_gpt2.rs:619-629, 2111) and trains from the loaded state:
