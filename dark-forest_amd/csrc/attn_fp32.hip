@@ -187,8 +187,6 @@ __global__ __launch_bounds__(64 * NW) void fwd_fp32_kernel(const float *__restri
   const int idx = __builtin_amdgcn_readfirstlane(linear_block() / H), head = linear_block() - idx * H;
   if (idx >= n_blocks) return;
   const Shape sh{S, D, H * D, head * D};
-  // Scores of hidden keys: their product with c2 must be -inf.
-  const float hidden = c2 < 0.f ? INFINITY : -INFINITY;
 
   // Longest query blocks first under causal masking; with `fold` the second
   // half of the workgroups takes the short blocks in ascending order.
@@ -232,37 +230,38 @@ __global__ __launch_bounds__(64 * NW) void fwd_fp32_kernel(const float *__restri
     for (int z = 0; z < KS; ++z)
       load_row_frags<DBLK>(K, (t + NW) * kTileKeys + kRows * z, sh, lane, kf[z]);
 
+    // P = 2^(s c2 - m); the exact column maximum and the rescale only when a
+    // score lies more than 8 above the reference point (or none is set). Keys are
+    // hidden after the scale is applied, which may be 0 (0 * inf is NaN).
     const bool masked = k0 + kTileKeys > n_clear;
-    if (masked) {
+    f32x4 x[KS];
+    auto exponents = [&](float ref) {
 #pragma unroll
       for (int z = 0; z < KS; ++z)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (k0 + kRows * z + 4 * g + r > lim) s[z][r] = hidden;
-    }
-    // P = 2^(s c2 - m); the exact column maximum and the rescale only when a
-    // score lies more than 8 above the reference point (or none is set).
+        for (int r = 0; r < 4; ++r) x[z][r] = fmaf(s[z][r], c2, -ref);
+      if (masked) {
+#pragma unroll
+        for (int z = 0; z < KS; ++z)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (k0 + kRows * z + 4 * g + r > lim) x[z][r] = -INFINITY;
+      }
+    };
     const float m_use = m == -INFINITY ? 0.f : m;
+    exponents(m_use);
     float top = -INFINITY;
-    f32x4 x[KS];
 #pragma unroll
     for (int z = 0; z < KS; ++z)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        x[z][r] = fmaf(s[z][r], c2, -m_use);
-        top = fmaxf(top, x[z][r]);
-      }
+      for (int r = 0; r < 4; ++r) top = fmaxf(top, x[z][r]);
     if (__any(top > 8.f || m == -INFINITY)) {
       const float m_new = fmaxf(m, m_use + column_max(top));
       const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - m_new);
-      const float use = m_new == -INFINITY ? 0.f : m_new;
       l *= alpha;
 #pragma unroll
       for (int b = 0; b < DBLK; ++b) acc[b] *= alpha;
-#pragma unroll
-      for (int z = 0; z < KS; ++z)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[z][r] = fmaf(s[z][r], c2, -use);
+      exponents(m_new == -INFINITY ? 0.f : m_new);
       m = m_new;
     }
 #pragma unroll

@@ -68,6 +68,18 @@ def test_scores_that_move_the_reference_point(device, scale):
     check(x, 2, scale, True, run(x, 2, scale, True, device))
 
 
+@pytest.mark.parametrize("d_head", [5, 64, 80, 128])
+@pytest.mark.parametrize("seq,causal", [(1, True), (40, True), (33, False), (48, False)])
+def test_scale_zero(device, d_head, seq, causal):
+    """Scale 0 weighs every visible key alike (and gives dQ and dK of zero); hidden keys, and those past a
+    ragged last tile, stay hidden."""
+    print(f"[gpu-fp32] scale 0 D={d_head} S={seq} causal={causal}", flush=True)
+    x = O.seeded_inputs(seq, 2, d_head, 60 + d_head)
+    got = run(x, 2, 0.0, causal, device, 1 if d_head == 64 else 0)
+    assert all(np.isfinite(t).all() for t in got.values())
+    check(x, 2, 0.0, causal, got)
+
+
 @pytest.mark.parametrize("d_head", [40, 128])
 def test_nonfinite_rows_stay_behind_the_mask(device, d_head):
     """Row 40 of V (then of dO) holds an infinity and a NaN: under causal masking no query before row
