@@ -165,8 +165,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_reg_kernel(float *logits, c
     }
     const float use = top == -INFINITY ? 0.f : top;  // no value yet: every term is 0
     s *= exp2f((m - use) * kLog2e);
-    m = top;
-    batch_m[b] = use;
+    m = batch_m[b] = top;
 #pragma unroll
     for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k)
 #pragma unroll
@@ -192,7 +191,8 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_reg_kernel(float *logits, c
   const float inv_sum = 1.f / tot;
 #pragma unroll
   for (int b = 0; b < kBatches; ++b) {
-    const float f = exp2f((batch_m[b] - row_m) * kLog2e) * inv_sum;
+    // (A batch without a value holds zeros about the stand-in 0, which may lie far above row_m.)
+    const float f = (batch_m[b] == -INFINITY ? 0.f : exp2f((batch_m[b] - row_m) * kLog2e)) * inv_sum;
 #pragma unroll
     for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k) {
       const int i = (tid + k * kCeThreads) * 4;

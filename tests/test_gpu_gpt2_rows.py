@@ -87,3 +87,36 @@ def test_cross_entropy_lengths(device, cols):
     assert (guard[:4] == 7).all() and (guard[4 + rows * cols:] == 7).all()
     ops.logit_ce_chunk(logits, targets.int(), logits, loss, 7)  # in place
     assert torch.equal(logits, grad)
+
+
+@pytest.mark.parametrize("cols", [16, 2048, 5000, 8192, 16384, 30000, 50257])
+def test_cross_entropy_masked_logits(device, cols):
+    """Logits of -inf (masked) in rows that lie far below and above zero: all the values that one thread
+    holds (four adjacent ones, again 2048 further), and all the first ones of every thread. A masked
+    logit's gradient is zero."""
+    import torch
+
+    print(f"[gpu-rows] cross-entropy masked cols={cols}", flush=True)
+    torch.manual_seed(cols)
+    rows, at = 5, torch.arange(cols, device=device)
+    logits = torch.randn(rows, cols, device=device)
+    logits += torch.tensor([-100.0, -300.0, 200.0, -1000.0, -100.0], device=device)[:, None]
+    one_thread = at // 4 % 512 == 1
+    first = at < min(10240, cols // 2)
+    for i, mask in enumerate((one_thread, first, first, at >= 0, one_thread | first)):
+        logits[i, mask] = float("-inf")
+    targets = torch.tensor([0, cols - 1, cols - 1, cols // 3, cols - 1], device=device)
+    logits[torch.arange(rows), targets] = torch.tensor([-101.0, -299.0, 201.0, -1000.0, -100.5], device=device)
+    want = torch.softmax(logits.double(), 1)
+    row_loss = -torch.log(want[torch.arange(rows), targets].clamp_min(1e-12)) / 7
+    masked = logits == float("-inf")
+    want[torch.arange(rows), targets] -= 1
+    grad, loss = torch.empty_like(logits), torch.empty(rows, device=device)
+    ops.logit_ce_chunk(logits, targets.int(), grad, loss, 7)
+    assert bool((grad[masked] == 0).all())
+    for i in (0, 1, 2, 4):
+        check(f"grad {i}", grad[i], want[i] / 7)
+    assert bool((grad[3] == 0).all())  # one value left: probability 1
+    assert float((loss - row_loss).abs().max()) <= 1e-5
+    ops.logit_ce_chunk(logits, targets.int(), logits, loss, 7)  # in place
+    assert torch.equal(logits, grad)
