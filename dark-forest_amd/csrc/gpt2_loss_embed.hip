@@ -175,7 +175,8 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_reg_kernel(float *logits, c
       }
   }
   const float wm = wave_max(m);
-  s = wave_sum(m == -INFINITY ? 0.f : s * exp2f((m - wm) * kLog2e));
+  // (A thread without a value holds 0, or NaN from logits that are NaN, which the maximum skips.)
+  s = wave_sum(m == -INFINITY ? s : s * exp2f((m - wm) * kLog2e));
   if (lane == 0) {
     red_m[wave] = wm;
     red_s[wave] = s;

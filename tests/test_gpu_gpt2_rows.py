@@ -120,3 +120,21 @@ def test_cross_entropy_masked_logits(device, cols):
     assert float((loss - row_loss).abs().max()) <= 1e-5
     ops.logit_ce_chunk(logits, targets.int(), logits, loss, 7)  # in place
     assert torch.equal(logits, grad)
+
+
+@pytest.mark.parametrize("cols", [16, 5000, 16384, 50257])
+def test_cross_entropy_nan_logits(device, cols):
+    """A NaN among the logits makes its row's gradient NaN, also where one thread holds nothing else, and
+    no other row's."""
+    import torch
+
+    print(f"[gpu-rows] cross-entropy NaN cols={cols}", flush=True)
+    torch.manual_seed(cols)
+    logits, at = torch.randn(4, cols, device=device), torch.arange(cols, device=device)
+    logits[0, cols // 2] = float("nan")
+    logits[1, at // 4 % 512 == 1] = float("nan")
+    logits[2, at // 4 % 512 == 1] = float("-inf")
+    logits[2, 5] = float("nan")
+    grad, loss = torch.empty_like(logits), torch.empty(4, device=device)
+    ops.logit_ce_chunk(logits, torch.zeros(4, dtype=torch.int32, device=device), grad, loss, 4)
+    assert bool(grad[:3].isnan().all()) and bool(grad[3].isfinite().all())
