@@ -2,8 +2,10 @@
 //
 // The reference's backward launchers take the caller's probability buffer,
 // which holds the row statistics that the fp32 kernels (attn_fp32.hip) need. A
-// NULL buffer, or a single-head one of one row (one float), is also accepted:
-// these calls take the kernel below, any d_head in 1..=128 in exact fp32, one
+// NULL buffer, or a single-head one of one row (one float), is also accepted.
+// And dfattn_bwd_main with an unaligned gradient must leave the workspace that
+// dfattn_bwd_preprocess filled for aligned tensors as it is. These calls take the
+// kernel below, any d_head in 1..=128 in exact fp32, one
 // wave per (query row, head); lanes take 64 keys at a time for the scores and
 // the d columns for the accumulations. Unlike the reference kernels
 // (attention_fused.cu:111-112, 417-420) it is correct for 64 < d_head <= 128

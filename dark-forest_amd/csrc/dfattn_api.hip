@@ -3,8 +3,8 @@
 //
 // Kernel selection: d_head == 64 with 16-byte aligned tensors takes the MFMA
 // kernels (attn_fwd_d64.hip, attn_bwd_d64.hip); every other valid shape takes
-// the fp32 kernels in attn_fp32.hip (or, for a backward launcher without
-// scratch, attn_generic.hip). There is no CPU path.
+// the fp32 kernels in attn_fp32.hip (or, for a backward without scratch of its
+// own, attn_generic.hip). There is no CPU path.
 #include <algorithm>
 #include <climits>
 #include <cstdio>
@@ -404,7 +404,9 @@ int dfattn_fwd_train(const float *q, const float *k, const float *v, float *o, f
 }
 
 // The split backward decides the fast path from q, k, v, o and d_o in both
-// phases, so main takes it only when preprocess filled the workspace.
+// phases, so main takes it only when preprocess filled the workspace. Main does
+// not write what preprocess filled: when only lse or a gradient is unaligned, it
+// takes the kernel that needs no workspace.
 int dfattn_bwd_preprocess(const float *q, const float *k, const float *v, const float *o,
                           const float *d_o, const float *lse, void *workspace, size_t workspace_bytes,
                           uint32_t n_heads, uint32_t seq_len, uint32_t d_head, float scale,
@@ -435,9 +437,13 @@ int dfattn_bwd_main(const float *q, const float *k, const float *v, const float 
   if (st != DFATTN_OK) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t err;
-  if (fast_path(d_head, {q, k, v, o, d_o}) && fast_path(d_head, {lse, d_q, d_k, d_v}))
+  const bool filled = fast_path(d_head, {q, k, v, o, d_o});
+  if (filled && fast_path(d_head, {lse, d_q, d_k, d_v}))
     err = dfattn::launch_bwd_main_d64(lse, d_q, d_k, d_v, workspace, (int)n_heads, (int)seq_len, scale,
                                       causal != 0, s);
+  else if (filled)
+    err = dfattn::launch_bwd_generic(q, k, v, d_o, d_q, d_k, d_v, (int)n_heads, (int)seq_len, (int)d_head,
+                                     scale, causal != 0, s);
   else
     err = dfattn::launch_bwd_fp32(q, k, v, o, d_o, lse, static_cast<float *>(workspace), d_q, d_k, d_v,
                                   (int)n_heads, (int)seq_len, (int)d_head, scale, causal != 0, s);

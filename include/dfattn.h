@@ -238,7 +238,9 @@ int dfattn_bwd(const float *q, const float *k, const float *v, const float *o,
  * separately (dfattn_bwd is exactly preprocess then main, on one stream,
  * with one workspace). Preprocess reads Q, K, V, O, dO and lse and fills
  * the workspace (row statistics and the fp16 operand copies); main reads
- * the workspace and writes dQ, dK, dV. Pass both phases the same
+ * the workspace and writes dQ, dK, dV (with d_head other than 64, or one of
+ * q, k, v, o and d_o not 16-byte aligned, preprocess has nothing to prepare
+ * and main uses the workspace as its scratch). Pass both phases the same
  * q, k, v, o, d_o, lse, workspace and scale. flags: 0, or
  * DFATTN_BWD_QKV_SAVED when a dfattn_fwd_train with the same q, k, v,
  * scale and workspace has run and neither q, k, v nor the workspace has

@@ -468,6 +468,31 @@ def test_split_backward_phases_match_dfattn_bwd(device):
         assert_close(f"split, unaligned o, {name}", host(a), host(b), scaled=True)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+def test_split_backward_main_leaves_the_workspace(device, causal):
+    """One preprocess serves several mains, also when a main between them writes gradients that are only
+    4-byte aligned (in fp32): the workspace stays as preprocess filled it."""
+    import torch
+
+    say(f"aligned, unaligned and aligned main after one preprocess, causal={causal}")
+    x = O.seeded_inputs(200, 3, 64, 3350)
+    q, k, v, g = (to_dev(x[n], device) for n in ("q", "k", "v", "do"))
+    o, lse = dfattn.attention_forward(q, k, v, 3, 0.125, causal)
+    ws = torch.full((dfattn.bwd_workspace_bytes(3, 200, 64) // 4,), float("nan"), device=device)
+    dfattn.backward_preprocess(q, k, v, o, g, lse, ws, 3, 0.125)
+    filled = ws.clone()
+    first, last = ([torch.empty_like(q) for _ in range(3)] for _ in range(2))
+    unaligned = [torch.empty(q.numel() + 1, device=device)[1:].view_as(q) for _ in range(3)]
+    for grads in (first, unaligned, last):
+        dfattn.backward_main(q, k, v, o, g, lse, *grads, ws, 3, 0.125, causal)
+    torch.cuda.synchronize()
+    assert torch.equal(ws.view(torch.int32), filled.view(torch.int32))
+    want = oracle_fwd_bwd(x, 3, 0.125, causal)
+    for name, a, b, c in zip(("dq", "dk", "dv"), first, unaligned, last):
+        assert torch.equal(a, c), name
+        assert_close(f"unaligned {name}", host(b), want[name], 2e-4, 1e-5)
+
+
 def test_training_forward_copies_match_the_full_conversion(device):
     """dfattn_fwd_train + preprocess(QKV_SAVED) + main give dfattn_fwd + dfattn_bwd's outputs bit for bit,
     causal and full, including a ragged length (rows past S are never written)."""
