@@ -36,6 +36,10 @@ namespace dfattn {
 namespace {
 
 constexpr int kRows = 16;  // rows of a tile
+// ln 2 - kLn2, so that lse = top * (kLn2 + kLn2Lo) + ln(sum) is rounded once, at
+// the end: 4.42e-8 from 64 bits on average over d_head 16 .. 128 at S = 64 .. 512,
+// 4.88e-8 with the log2 domain's sum times kLn2.
+constexpr float kLn2Lo = -1.90465421e-09f;
 
 // fp32 vectors at any 4-byte alignment.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -330,7 +334,7 @@ __global__ __launch_bounds__(64 * NW) void fwd_fp32_kernel(const float *__restri
         if (d < D) row[d] = o[r] * inv;
       }
       if (LSE != nullptr && b == 0 && g == 0)
-        LSE[(size_t)head * S + q] = sum > 0.f ? (top + __builtin_log2f(sum)) * kLn2 : -INFINITY;
+        LSE[(size_t)head * S + q] = sum > 0.f ? fmaf(top, kLn2, fmaf(top, kLn2Lo, logf(sum))) : -INFINITY;
     }
   }
 }
