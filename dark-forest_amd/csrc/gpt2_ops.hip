@@ -366,10 +366,12 @@ __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restric
   const int col = strip * kColStrip + 4 * c4;
   float4 a0 = splat4(0.f), a1 = splat4(0.f);
   if (col < cols) {
-    int r = slot;
+    // (Unsigned: the step past the last row may pass 2^31.)
+    unsigned r = slot;
+    const unsigned n_rows = rows;
     if constexpr (!LN) {
       // kColAhead rows' loads in flight per thread, then their sums in order.
-      for (; r + (kColAhead - 1) * kRowSlots < rows; r += kColAhead * kRowSlots) {
+      for (; r + (kColAhead - 1) * kRowSlots < n_rows; r += kColAhead * kRowSlots) {
         float4 v[kColAhead];
 #pragma unroll
         for (int k = 0; k < kColAhead; ++k)
@@ -384,7 +386,7 @@ __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restric
       }
     }
 #pragma unroll 4
-    for (; r < rows; r += kRowSlots) {
+    for (; r < n_rows; r += kRowSlots) {
       const float4 gv = *reinterpret_cast<const float4 *>(g + (size_t)r * cols + col);
       if constexpr (LN) {
         const float4 xv = *reinterpret_cast<const float4 *>(x + (size_t)r * cols + col);

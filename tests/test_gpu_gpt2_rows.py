@@ -62,6 +62,22 @@ def test_bias_gradient_row_blocks(device, rows):
     check("bias", ops.bias_grad(g), g.double().sum(0))
 
 
+def test_bias_gradient_of_the_most_rows(device):
+    """2^31 - 1 rows of four ones: a row slot's index ends next to 2^31. Each of the 256 slots counts 2^23
+    rows (one a row less), exactly; their total rounds to 2^31."""
+    import torch
+
+    rows = 2 ** 31 - 1
+    if torch.cuda.mem_get_info()[0] < rows * 16 + (4 << 30):
+        pytest.skip("needs 36 GiB of free device memory")
+    print(f"[gpu-rows] bias gradient rows={rows}", flush=True)
+    g = torch.ones(rows, 4, device=device)
+    got = ops.bias_grad(g).tolist()
+    del g
+    torch.cuda.empty_cache()
+    assert got == [2.0 ** 31] * 4
+
+
 @pytest.mark.parametrize("cols", [1, 3, 2047, 2048, 2049, 8192, 8195, 16384, 16385, 30720, 30721, 50257, 51200, 51201])
 def test_cross_entropy_lengths(device, cols):
     """One row all -1e30 but its target, and one whose largest logit comes last."""
