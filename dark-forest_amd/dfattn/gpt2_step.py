@@ -86,6 +86,7 @@ def tune_gemms(path=GEMM_SOLUTIONS, seq_len=1024, steps=2, seed=0):
     torch = _torch()
     tun = torch.cuda.tunable
     model = StaticGPT2(seq_len=seq_len, seed=seed, tuned_gemms=False)
+    model._engine.library_products = True  # also at the sizes where dfgpt2_linear_* are the faster ones
     tokens, targets = synthetic_batch(model.vocab_size, seq_len, 1, model.device)
     prev = tun.is_enabled(), tun.tuning_is_enabled()
     tun.set_filename(os.devnull)  # TunableOp's own write at exit; the file is written below
@@ -306,6 +307,7 @@ class _NativeEngine:
         torch = _torch()
         self.m = weakref.proxy(m)  # no cycle: a model's memory and graph go with its last reference
         self.exact_sites = dict(self.EXACT_SITES)
+        self.library_products = False  # every product on hipBLASLt / rocBLAS, whatever _own_gemms' sizes say
         S, d, F, V, L, H = m.seq_len, m.d_model, m.d_ff, m.vocab_size, m.n_layers, m.n_heads
         self.chunk = min(S, 512)  # static_gpt2.rs:423
         dev = m.device
@@ -422,6 +424,8 @@ class _NativeEngine:
         past it the library's larger tiles win (2048 rows: qkv_fwd 37 and 48). All of a step or
         none, because these kernels fill a CU's LDS and gain nothing from a second stream: the whole
         step takes 6.51 ms on one stream, 6.99 on two; on hipBLASLt 6.99 and 6.74."""
+        if self.library_products:
+            return False
         S, d, F = self.m.seq_len, self.m.d_model, self.m.d_ff
         products = ((S, 3 * d), (S, F), (d, F), (F, d), (3 * d, d), (S, d))
         return self.m.fast_gemm and max(-(-r // 128) * -(-c // 96) for r, c in products) <= 256
