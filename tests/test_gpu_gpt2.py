@@ -126,6 +126,36 @@ def test_captured_step_replays_match_eager_steps(device):
         assert torch.allclose(a, b, rtol=0, atol=1e-6)
 
 
+@pytest.mark.parametrize("cfg", [
+    dict(vocab_size=500, d_model=128, n_heads=2, n_layers=3, d_ff=512, seq_len=256, fast_gemm=False),
+    # 9 x 32 tiles of 128 x 96: one row past the sizes whose fast products are the engine's own
+    dict(vocab_size=500, d_model=768, n_heads=12, n_layers=2, d_ff=3072, seq_len=1025),
+    dict(vocab_size=500, d_model=768, n_heads=12, n_layers=2, d_ff=3072, seq_len=1024)])
+def test_captured_step_on_library_and_own_products(device, cfg):
+    """Eager steps against replayed ones where the recorded weight gradients run on a second stream (every
+    product on the library: exact ones, or fast ones at sizes past the rule), and at the rule's last size,
+    where they do not."""
+    import torch
+
+    own = cfg["seq_len"] == 1024
+    say(f"captured step, {'own' if own else 'library'} products: {cfg}")
+    eager, graph = (StaticGPT2(**cfg, lr=1e-3, seed=4, capturable=True) for _ in range(2))
+    assert graph._engine._own_gemms() == own
+    tokens, targets = synthetic_batch(cfg["vocab_size"], cfg["seq_len"], 13, device)
+    want = [float(eager.step(tokens, targets)) for _ in range(5)]
+    loss = graph.capture(tokens, targets, warmup=2)
+    assert graph._engine._overlap == (not own)
+    for i in range(2, 5):
+        graph.replay()
+        torch.cuda.synchronize()
+        got = float(loss)
+        _ = torch.ones(4096, device=device).sum().item()
+        say(f"replay {i}: graph {got:.7f} eager {want[i]:.7f}")
+        assert abs(got - want[i]) <= 1e-6 * abs(want[i])
+    for a, b in zip(eager.parameters(), graph.parameters()):
+        assert torch.allclose(a, b, rtol=0, atol=1e-6)
+
+
 def test_capture_frees_models_out_of_use_before_recording(device):
     """A captured model that went out of use is freed before another one's recording starts: the cycle
     collector, run inside the recording, finds none (freeing a recorded graph there ends the process)."""

@@ -95,3 +95,21 @@ def test_step_with_own_and_library_products(device):
     assert abs(float(own.step(tokens, targets)) - float(exact.step(tokens, targets))) < 1e-4
     g, ref = own.opt.arena.g, exact.opt.arena.g
     assert float((g - ref).norm() / ref.norm()) < 1e-4
+
+
+def test_step_with_library_products_at_the_fast_sites(device):
+    """The same step with the fast sites on hipBLASLt's fast path (first MLP bias and GELU in a kernel of
+    their own, GELU's derivative after the product): the same values to the fast paths' error."""
+    import torch
+
+    from dfattn.gpt2_step import StaticGPT2, synthetic_batch
+
+    cfg = dict(vocab_size=500, d_model=96, n_heads=3, n_layers=2, d_ff=384, seq_len=130, seed=4)
+    tokens, targets = synthetic_batch(500, 130, 5, device)
+    print("[gpu-linear] GPT-2 step: own and library fast products", flush=True)
+    own, library = StaticGPT2(**cfg), StaticGPT2(**cfg)
+    library._engine.library_products = True
+    assert own._engine._own_gemms() and not library._engine._own_gemms()
+    assert abs(float(own.step(tokens, targets)) - float(library.step(tokens, targets))) < 1e-4
+    g, ref = own.opt.arena.g, library.opt.arena.g
+    assert float((g - ref).norm() / ref.norm()) < 1e-4

@@ -20,15 +20,15 @@ def check(name, got, want, rel=6e-6):
     assert err <= rel and worst <= 1e-4, f"{name}: rel {err:.1e}, max {worst:.1e}"
 
 
-@pytest.mark.parametrize("rows,features", [(1, 1028), (5, 1536), (7, 1600), (2051, 2048), (4097, 768), (8200, 1024),
-                                           (9, 2052), (6, 1030)])
-@pytest.mark.parametrize("workspace", [True, False])
+WIDE_ROWS = [(1, 1028), (5, 1536), (7, 1600), (2051, 2048), (9, 2052), (6, 1030)]
+
+
+@pytest.mark.parametrize("rows,features,workspace", [(*s, True) for s in WIDE_ROWS + [(4097, 768), (8200, 1024)]] +
+                         [(*s, False) for s in WIDE_ROWS])
 def test_layer_norm_widths(device, rows, features, workspace):
     """With and without a workspace: only rows of at most 1024 features need one."""
     import torch
 
-    if not workspace and features <= 1024:
-        pytest.skip("needs its workspace")
     print(f"[gpu-rows] LayerNorm {rows} x {features} workspace={workspace}", flush=True)
     torch.manual_seed(rows + features)
     x, y, dy, res = (torch.randn(rows, features, device=device) for _ in range(4))

@@ -343,16 +343,18 @@ def test_legacy_mha_launchers_match_fast_path(device):
             {n: want[n] for n in ("o", "dq", "dk", "dv")}, scaled=True)
 
 
-def test_legacy_backward_with_small_scratch_uses_generic_kernel(device):
-    """S=8 < the fast path's workspace needs: the self-contained fp32 kernel runs."""
-    say("legacy backward, tiny scratch")
+@pytest.mark.parametrize("scratch", [True, False])
+def test_legacy_backward_with_small_scratch_uses_generic_kernel(device, scratch):
+    """S=8 < the fast path's workspace needs: the fp32 kernels run, and with a NULL scratch the
+    self-contained one."""
+    say(f"legacy backward, tiny scratch {scratch}")
     import torch
 
     h, s, d = 2, 8, 64
     x = O.seeded_inputs(s, h, d, 8100)
     q, k, v, g = (to_dev(x[n], device) for n in ("q", "k", "v", "do"))
     dq, dk, dv = (torch.zeros_like(q) for _ in range(3))
-    probs = torch.empty(h * 2 * s * s, dtype=torch.float32, device=device)
+    probs = torch.empty(h * 2 * s * s, dtype=torch.float32, device=device) if scratch else None
     dfattn.launch_fused_mha_backward(q, k, v, g, dq, dk, dv, probs, h, s, d, 0.125, True)
     dfattn.darkforest_sync()
     want = oracle_fwd_bwd(x, h, 0.125, True)
