@@ -114,23 +114,31 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_kernel(float *logits, const
   }
 }
 
-// The same contract with the row held in registers, K4 groups of four values
-// per thread (cols <= 4 * K4 * kCeThreads): one read and one write of the row.
-// What bounds it is HBM, as long as the arithmetic runs beside the loads and
-// stores: every load is issued first, and as the values arrive, kCeBatch groups
-// at a time, they become exponentials about the thread's maximum so far. The
-// threads' (max, sum) merge in a fixed order (lanes by butterfly, then the
-// waves in order), and each batch's exponentials are scaled to the row's
+// The same contract with the row held in registers, K4 groups of W values (four,
+// or one for rows of at most kCeThreads) per thread (cols <= W * K4 *
+// kCeThreads): one read and one write of the row.
+// Every load is issued first, and sums merge in a fixed order (lanes by
+// butterfly, then the waves in order).
+// Long rows (K4 > 8): what bounds them is HBM, as long as the arithmetic runs
+// beside the loads and stores. As the values arrive, kCeBatch groups at a time,
+// they become exponentials about the thread's maximum so far; the threads'
+// (max, sum) merge, and each batch's exponentials are scaled to the row's
 // maximum and sum as they are stored. (With one exponential pass between a row
 // maximum and the stores, and 4-byte accesses, all workgroups computed at once
 // and the memory idled: 512 rows of 50257 took 41.9 us, now 30.9 us, 6.7 TB/s of
-// reads and writes that the Infinity Cache holds; 512 of 8000 9.4, now 7.4.)
+// reads and writes that the Infinity Cache holds.)
+// Shorter rows: latency, so the row's maximum first and then one exponential a
+// value, a barrier more and a chain of rescaling exponentials less, and no more
+// groups than the row fills. 1024 rows, us, this against the scheme of long rows
+// with four or eight groups: 2049 values 5.9 and 8.6, 4096 7.4 and 10.1; 512 rows
+// of 9000 9.2 and 10.4; one value a thread against four: 1024 rows of 512 4.2 and
+// 4.6.
 // A row starts at any 4-byte address: 16-byte buffer accesses need no more
 // alignment than that, and their bounds are checked value by value.
 constexpr int kCeBatch = 5;
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-template <bool WRITE_PROBS, bool ROW_LOSS, int K4>
+template <bool WRITE_PROBS, bool ROW_LOSS, int K4, int W>
 __global__ __launch_bounds__(kCeThreads) void ce_row_reg_kernel(float *logits, const uint32_t *__restrict__ targets,
                                                                 float *grad, float *__restrict__ row_loss,
                                                                 float *__restrict__ loss, int cols, float inv_total) {
@@ -145,63 +153,111 @@ __global__ __launch_bounds__(kCeThreads) void ce_row_reg_kernel(float *logits, c
   const float xt = (tid == 0 && target < (uint32_t)cols) ? x[target] : -INFINITY;
   const auto rx = buffer_rsrc(x, (unsigned)cols * 4u);
   const auto rg = buffer_rsrc(gx, (unsigned)cols * 4u);
-  f32x4 v[K4];
+  typedef float group_t __attribute__((ext_vector_type(W)));
+  group_t v[K4];
 #pragma unroll
-  for (int k = 0; k < K4; ++k)
-    v[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (tid + k * kCeThreads) * 16, 0, 0));
-  float m = -INFINITY, s = 0.f;
-  float batch_m[kBatches];
+  for (int k = 0; k < K4; ++k) {
+    const int at = (tid + k * kCeThreads) * W * 4;
+    if constexpr (W == 4)
+      v[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, at, 0, 0));
+    else
+      v[k][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, at, 0, 0));
+  }
+  auto mask = [&](int k) {
+    if ((k + 1) * kCeThreads * W > cols) {
 #pragma unroll
-  for (int b = 0; b < kBatches; ++b) {
-    float top = m;
-#pragma unroll
-    for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k) {
-      if ((k + 1) * kCeThreads * 4 > cols) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if ((tid + k * kCeThreads) * 4 + j >= cols) v[k][j] = -INFINITY;
-      }
-      top = fmaxf(top, fmaxf(fmaxf(v[k][0], v[k][1]), fmaxf(v[k][2], v[k][3])));
+      for (int j = 0; j < W; ++j)
+        if ((tid + k * kCeThreads) * W + j >= cols) v[k][j] = -INFINITY;
     }
-    const float use = top == -INFINITY ? 0.f : top;  // no value yet: every term is 0
-    s *= exp2f((m - use) * kLog2e);
-    m = batch_m[b] = top;
+  };
+  auto group_max = [&](int k) {
+    if constexpr (W == 1) return v[k][0];
+    return fmaxf(fmaxf(v[k][0], v[k][1 % W]), fmaxf(v[k][2 % W], v[k][3 % W]));
+  };
+  auto store = [&](auto rs, int i, group_t x) {
+    if constexpr (W == 4)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, i * 4, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x[0]), rs, i * 4, 0, 0);
+  };
+  auto write = [&](int k, float f) {
+    const int i = (tid + k * kCeThreads) * W;
+    group_t p = v[k] * f, gv;
 #pragma unroll
-    for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k)
+    for (int j = 0; j < W; ++j) gv[j] = (p[j] - ((uint32_t)(i + j) == target ? 1.f : 0.f)) * inv_total;
+    if (WRITE_PROBS) store(rx, i, p);
+    store(rg, i, gv);
+  };
+  float m = -INFINITY, s = 0.f, row_m, tot = 0.f, inv_sum;
+  if constexpr (K4 <= 8) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[k][j] = exp2f((v[k][j] - use) * kLog2e);  // 0 past the row's end
+    for (int k = 0; k < K4; ++k) {
+      mask(k);
+      m = fmaxf(m, group_max(k));
+    }
+    m = wave_max(m);
+    if (lane == 0) red_m[wave] = m;
+    __syncthreads();
+    row_m = red_m[0];
+#pragma unroll
+    for (int w = 1; w < kCeThreads / 64; ++w) row_m = fmaxf(row_m, red_m[w]);
+#pragma unroll
+    for (int k = 0; k < K4; ++k)
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        v[k][j] = exp2f((v[k][j] - row_m) * kLog2e);  // 0 past the row's end
         s += v[k][j];
       }
-  }
-  const float wm = wave_max(m);
-  // (A thread without a value holds 0, or NaN from logits that are NaN, which the maximum skips.)
-  s = wave_sum(m == -INFINITY ? s : s * exp2f((m - wm) * kLog2e));
-  if (lane == 0) {
-    red_m[wave] = wm;
-    red_s[wave] = s;
-  }
-  __syncthreads();
-  float row_m = red_m[0];
+    s = wave_sum(s);
+    if (lane == 0) red_s[wave] = s;
+    __syncthreads();
 #pragma unroll
-  for (int w = 1; w < kCeThreads / 64; ++w) row_m = fmaxf(row_m, red_m[w]);
-  float tot = 0.f;
+    for (int w = 0; w < kCeThreads / 64; ++w) tot += red_s[w];
+    inv_sum = 1.f / tot;
 #pragma unroll
-  for (int w = 0; w < kCeThreads / 64; ++w)
-    tot += red_m[w] == -INFINITY ? red_s[w] : red_s[w] * exp2f((red_m[w] - row_m) * kLog2e);
-  const float inv_sum = 1.f / tot;
+    for (int k = 0; k < K4; ++k) write(k, inv_sum);
+  } else {
+    float batch_m[kBatches];
 #pragma unroll
-  for (int b = 0; b < kBatches; ++b) {
-    // (A batch without a value holds zeros about the stand-in 0, which may lie far above row_m.)
-    const float f = (batch_m[b] == -INFINITY ? 0.f : exp2f((batch_m[b] - row_m) * kLog2e)) * inv_sum;
+    for (int b = 0; b < kBatches; ++b) {
+      float top = m;
 #pragma unroll
-    for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k) {
-      const int i = (tid + k * kCeThreads) * 4;
-      f32x4 p = v[k] * f, gv;
+      for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k) {
+        mask(k);
+        top = fmaxf(top, group_max(k));
+      }
+      const float use = top == -INFINITY ? 0.f : top;  // no value yet: every term is 0
+      s *= exp2f((m - use) * kLog2e);
+      m = batch_m[b] = top;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) gv[j] = (p[j] - ((uint32_t)(i + j) == target ? 1.f : 0.f)) * inv_total;
-      if (WRITE_PROBS) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, p), rx, i * 4, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, gv), rg, i * 4, 0, 0);
+      for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k)
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+          v[k][j] = exp2f((v[k][j] - use) * kLog2e);  // 0 past the row's end
+          s += v[k][j];
+        }
+    }
+    const float wm = wave_max(m);
+    // (A thread without a value holds 0, or NaN from logits that are NaN, which the maximum skips.)
+    s = wave_sum(m == -INFINITY ? s : s * exp2f((m - wm) * kLog2e));
+    if (lane == 0) {
+      red_m[wave] = wm;
+      red_s[wave] = s;
+    }
+    __syncthreads();
+    row_m = red_m[0];
+#pragma unroll
+    for (int w = 1; w < kCeThreads / 64; ++w) row_m = fmaxf(row_m, red_m[w]);
+#pragma unroll
+    for (int w = 0; w < kCeThreads / 64; ++w)
+      tot += red_m[w] == -INFINITY ? red_s[w] : red_s[w] * exp2f((red_m[w] - row_m) * kLog2e);
+    inv_sum = 1.f / tot;
+#pragma unroll
+    for (int b = 0; b < kBatches; ++b) {
+      // (A batch without a value holds zeros about the stand-in 0, which may lie far above row_m.)
+      const float f = (batch_m[b] == -INFINITY ? 0.f : exp2f((batch_m[b] - row_m) * kLog2e)) * inv_sum;
+#pragma unroll
+      for (int k = b * kCeBatch; k < K4 && k < (b + 1) * kCeBatch; ++k) write(k, f);
     }
   }
   if (tid == 0) {
@@ -222,12 +278,17 @@ void launch_ce(float *logits, const uint32_t *targets, float *grad, float *row_l
                uint32_t cols, float inv_total, hipStream_t stream) {
   const dim3 grid(rows), block(kCeThreads);
   const int c = (int)cols;
-  auto in_registers = [&](auto k4) {
-    hipLaunchKernelGGL((ce_row_reg_kernel<WRITE_PROBS, ROW_LOSS, decltype(k4)::value>), grid, block, 0, stream,
+  auto in_registers = [&](auto k4, auto... w) {
+    constexpr int W = sizeof...(w) ? 1 : 4;
+    hipLaunchKernelGGL((ce_row_reg_kernel<WRITE_PROBS, ROW_LOSS, decltype(k4)::value, W>), grid, block, 0, stream,
                        logits, targets, grad, row_loss, loss, c, inv_total);
   };
-  if (cols <= 4u * kCeThreads)
+  if (cols <= 1u * kCeThreads)
+    in_registers(std::integral_constant<int, 1>{}, 1);
+  else if (cols <= 4u * kCeThreads)
     in_registers(std::integral_constant<int, 1>{});
+  else if (cols <= 8u * kCeThreads)
+    in_registers(std::integral_constant<int, 2>{});
   else if (cols <= 16u * kCeThreads)
     in_registers(std::integral_constant<int, 4>{});
   else if (cols <= 32u * kCeThreads)

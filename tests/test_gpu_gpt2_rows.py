@@ -78,7 +78,7 @@ def test_bias_gradient_of_the_most_rows(device):
     assert got == [2.0 ** 31] * 4
 
 
-@pytest.mark.parametrize("cols", [1, 3, 2047, 2048, 2049, 8192, 8195, 16384, 16385, 30720, 30721, 50257, 51200, 51201])
+@pytest.mark.parametrize("cols", [1, 3, 511, 512, 513, 2047, 2048, 2049, 4096, 4097, 8192, 8195, 16384, 16385, 30720, 30721, 50257, 51200, 51201])
 def test_cross_entropy_lengths(device, cols):
     """One row all -1e30 but its target, and one whose largest logit comes last."""
     import torch
@@ -105,7 +105,7 @@ def test_cross_entropy_lengths(device, cols):
     assert torch.equal(logits, grad)
 
 
-@pytest.mark.parametrize("cols", [16, 2048, 5000, 8192, 16384, 30000, 50257])
+@pytest.mark.parametrize("cols", [16, 2048, 3000, 5000, 8192, 16384, 30000, 50257])
 def test_cross_entropy_masked_logits(device, cols):
     """Logits of -inf (masked) in rows that lie far below and above zero: all the values that one thread
     holds (four adjacent ones, again 2048 further), and all the first ones of every thread. A masked
