@@ -1328,8 +1328,11 @@ void build_xcd_order(Sched &sched, int n_heads) {
 // Measured, short against the other, us: H = 12 causal S = 128 5.9 / 6.9, 512 9.1
 // / 12.1, 1024 16.0 / 18.4, 2048 39.8 / 33.7; unmasked 512 10.4 / 11.3, 1024
 // 25.3 / 18.3; H = 4 causal 2048 19.3 / 29.1, 4096 52.2 / 54.4; H = 1 4096 25.5 /
-// 50.7; H = 16 1024 20.3 / 19.8 (the other).
+// 50.7; H = 16 1024 20.3 / 19.8 (the other). Without masking all workgroups are
+// equally long, and a few more than 512 (two a CU) take a second round: H = 4 2049
+// 35.9 / 29.9 (the other).
 static bool bwd_short(int n_heads, int seq_len, bool causal) {
+  if (!causal && 2LL * n_heads * ((seq_len + kShortRows - 1) / kShortRows) > 512) return false;
   const double nb = (seq_len + kShortRows - 1) / kShortRows, n64 = (seq_len + kQBlock - 1) / kQBlock;
   const double tiles = 2.0 * n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb);
   return tiles * 215 / 256 < n64 * 870;

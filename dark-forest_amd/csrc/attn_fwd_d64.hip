@@ -823,10 +823,18 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void fwd_d64_short_kernel(
 // 10.0, 1024 10.3 / 14.1, 1536 15.2 / 17.8, 2048 25.3 / 22.7 (staged); unmasked
 // 512 7.2 / 11.6, 1536 28.8 / 19.8 (staged); H = 16 causal 1024 10.8 / 14.3, 2048
 // 30.3 / 23.2 (staged); H = 4 causal 4096 28.3 / 35.2; H = 1 4096 24.7 / 34.6.
+// A causal grid of more than 512 workgroups (two a CU, see fold) fills its second
+// round badly: 10 % more per tile, and 15 ns for each workgroup past them. H = 14
+// causal 1537 22.6 / 20.2, H = 5 4500 44.5 / 40.4, H = 7 3072 33.1 / 30.9 (all
+// staged); H = 12 1537 18.0 / 19.6, H = 16 1150 16.0 / 17.2. Over H = 1 .. 16 and S
+// = 256 .. 8192 the choice is at most 6 % slower than the staged kernel (H = 7
+// unmasked 1537, H = 11 causal 1700), most often at odd head counts.
 bool fwd_short(int n_heads, int seq_len, bool causal) {
   const long long nb = (seq_len + kShortRows - 1) / kShortRows, n64 = (seq_len + kBN - 1) / kBN;
-  const long long tiles = n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb);
-  return std::max(tiles * 200 / 256, nb * 620 / kShortWaves) < n64 * 566;
+  const long long tiles = n_heads * (causal ? nb * (nb + 1) / 2 : nb * nb), n_wg = nb * n_heads;
+  const bool round2 = causal && n_wg > 512;
+  const long long short_ns = tiles * (round2 ? 220 : 200) / 256 + (round2 ? 15 * (n_wg - 512) : 0);
+  return std::max(short_ns, nb * 620 / kShortWaves) < n64 * 566;
 }
 
 }  // namespace

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("n_heads,seq", [(1, 1), (2, 31), (2, 32), (2, 33), (3, 63), (3, 64), (2, 95), (2, 97), (3, 128),
-                                         (3, 129), (2, 161), (12, 545)])
+                                         (3, 129), (2, 161), (12, 545), (12, 1409)])
 def test_short(device, n_heads, seq, causal):
     say(f"short H={n_heads} S={seq} causal={causal}")
     x = O.seeded_inputs(seq, n_heads, 64, 600 + seq)
@@ -20,7 +20,8 @@ def test_short(device, n_heads, seq, causal):
     compare("pair", run_training_pair(x, n_heads, 0.125, causal, device), want, scaled=True)
 
 
-@pytest.mark.parametrize("n_heads,seq,causal", [(16, 2047, True), (16, 2049, True), (16, 2175, True), (16, 1537, False)])
+@pytest.mark.parametrize("n_heads,seq,causal", [(16, 2047, True), (16, 2049, True), (16, 2175, True), (16, 1537, False),
+                                                (14, 1537, True), (4, 2049, False)])
 def test_staged(device, n_heads, seq, causal):
     say(f"staged H={n_heads} S={seq} causal={causal}")
     x = O.seeded_inputs(seq, n_heads, 64, 700 + seq)
