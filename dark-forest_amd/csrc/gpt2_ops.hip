@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_generic_kernel(const float *__r
 // added in order through LDS, into partial[blockIdx.x][plane][features].
 // colsum_partials_kernel adds the workgroups' partials in order. The rows are
 // read once for all of it.
-template <int V>
+template <int V, bool ONE>
 __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const float *__restrict__ dout, const float *__restrict__ x,
                                                            const float *__restrict__ gamma,
                                                            const float *__restrict__ means,
@@ -239,6 +239,7 @@ __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const float *__restri
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[p][i] = splat4(0.f);
   auto add = [](float4 &a, float4 b) { a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+  if (ONE) rows_per_wave = 1;
   for (int k = 0; k < rows_per_wave; ++k) {
     const unsigned row = (blockIdx.x * rows_per_wave + k) * 4u + wave;
     if (row >= (unsigned)batch) break;
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(1024) void colsum_vec_kernel(const float *__restric
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int slot = 16 * w + (lane >> 2);
   const int c4 = lane & 3;
-  const int strip = strip_of(blockIdx.x, gridDim.x);
+  const int strip = strip_of(blockIdx.x, (cols + kColStrip - 1) / kColStrip);
   const int col = strip * kColStrip + 4 * c4;
   float4 a0 = splat4(0.f), a1 = splat4(0.f);
   if (col < cols) {
@@ -685,8 +686,9 @@ void ln_backward_dx(const float *dout, const float *x, const float *gamma, const
                     const float *residual, float *grad_x, int b, int f, hipStream_t stream);
 
 // The register-resident row path: features % 4 == 0, at most 2048 (8 float4 a
-// lane: with its column sums the backward then takes 200 of the 256 registers
-// of two waves per SIMD), 16-byte aligned tensors. Above 1024 features rows used
+// lane: with its column sums the backward then takes 206 registers, and its merge
+// 96 KB of LDS, so one workgroup a CU; 72 KB and two up to 1536), 16-byte aligned
+// tensors. Above 1024 features rows used
 // to take the generic path, three reads of the row: at 8192 x 2048 add+LayerNorm
 // took 76 us and its backward 133 us, now 42 and 97.
 bool ln_vec(uint32_t features, std::initializer_list<const void *> ptrs) {
@@ -850,12 +852,20 @@ extern "C" int dfgpt2_layernorm_backward_fused(const float *grad_out, const floa
                                                   std::to_string(need) + " bytes");
   float *partial = static_cast<float *>(workspace);
   // More rows per wave mean fewer partial sums to write and add up, as long as
-  // 512 workgroups remain (two per CU).
+  // 512 workgroups remain: two rounds of the widest rows' one workgroup a CU, all
+  // at once up to 1536 features. (One row needs no sums over rows: 22-53 registers
+  // less, and 768 features over 128 rows take 6.9 us in place of 7.2.)
   const int rows_per_wave = std::max(1, std::min(8, b / (4 * 512)));
   const int n_parts = (b + 4 * rows_per_wave - 1) / (4 * rows_per_wave);
   with_ln_vectors(f, [&](auto v) {
-    hipLaunchKernelGGL(ln_bwd_fused_kernel<decltype(v)::value>, dim3(n_parts), dim3(256), 0, stream, grad_out, x, gamma,
-                       means, rstds, residual, grad_x, partial, planes, b, f, rows_per_wave);
+    auto launch = [&](auto *kernel) {
+      hipLaunchKernelGGL(kernel, dim3(n_parts), dim3(256), 0, stream, grad_out, x, gamma, means, rstds, residual,
+                         grad_x, partial, planes, b, f, rows_per_wave);
+    };
+    if (rows_per_wave == 1)
+      launch(ln_bwd_fused_kernel<decltype(v)::value, true>);
+    else
+      launch(ln_bwd_fused_kernel<decltype(v)::value, false>);
   });
   if (int st = launched(fn); st != DFATTN_OK) return st;
   hipLaunchKernelGGL(colsum_partials_kernel, dim3((planes * f + 15) / 16), dim3(256), 0, stream, partial, n_parts,
