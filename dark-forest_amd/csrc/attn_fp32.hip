@@ -169,8 +169,8 @@ __device__ __forceinline__ bool any_nonfinite(const T (&f)[N]) {
 // product, V of this one during the first. The online softmax works in the
 // log2 domain and moves its reference point only when a score exceeds it by
 // more than 8 (P stays below 2^8, the sums are fp32). Four waves a workgroup:
-// three workgroups share a CU, so that one's loads and merge run beside
-// another's products (eight waves measured 15-25 % slower at S = 1000).
+// three workgroups share a CU (two above d_head 96), so that one's loads and merge
+// run beside another's products (eight waves measured 15-25 % slower at S = 1000).
 // Measured: H = 12, S = 1000, d_head 80 causal 29.4 us (607 us with one wave
 // per row on the vector unit); H = 8, d_head 128: S = 1024 causal 29.1 us (620
 // us), S = 4096 full 592 us = 116 TFLOP/s of the 157 the fp32 MFMA has (537 us
@@ -589,8 +589,8 @@ hipError_t launch_fwd_fp32(const float *q, const float *k, const float *v, float
     constexpr int DBLK = decltype(n)::value, KS = DBLK <= 4 ? 2 : 1, NW = 4;
     const int n_blocks = (seq_len + kRows - 1) / kRows;
     const size_t grid = (size_t)n_blocks * n_heads;
-    // When every workgroup is resident at once (three per CU on 256 CUs) there
-    // is no later round to fill the gaps of the long ones: the short half in
+    // When every workgroup is resident at once (three per CU on 256 CUs up to
+    // d_head 96, two above) there is no later round to fill the gaps of the long ones: the short half in
     // ascending order then lands beside them (29.1 against 34.9 us at H = 8, S =
     // 1024, d_head 128). Larger grids run longest first (94 against 107 us at S
     // = 2048).

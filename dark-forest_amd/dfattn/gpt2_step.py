@@ -57,7 +57,8 @@ def _f32(x):
 
 
 # GEMM solutions PyTorch's TunableOp measured fastest for the engine's GEMM shapes (GPT-2 small, S =
-# 1024) on MI355X with this image's PyTorch, HIP, hipBLASLt and rocBLAS (written by tune_gemms). Each
+# 1024) on MI355X with this image's PyTorch, HIP, hipBLASLt and rocBLAS (written by tune_gemms). The fast
+# linear-layer shapes among them serve a model of those widths that is past _own_gemms' sizes. Each
 # call keeps its math mode: the fast fp32 call sites choose among hipBLASLt's fast fp32 solutions,
 # the exact ones among exact fp32 solutions (rocBLAS or hipBLASLt). The file's validators make
 # TunableOp ignore it under other library versions or GPUs, shapes it does not list keep the
@@ -418,10 +419,14 @@ class _NativeEngine:
     def _own_gemms(self):
         """Whether the step's fast sites run on dfgpt2_linear_* (the fast path's accuracy) rather than
         on hipBLASLt: while the largest of their products is at most one 128 x 96 tile per CU. Up to
-        there they measured faster at every size and site (us in a graph, hipBLASLt first, GPT-2
-        small's widths: fc1_fwd 25.2 and 24.9 with its bias and GELU still to come for hipBLASLt,
-        qkv_fwd 25.0 and 23.7, qkv_dw 29.7 and 21.0, wo_dx 15.2 and 10.3; at 64 rows 11.1 and 9.9);
-        past it the library's larger tiles win (2048 rows: qkv_fwd 37 and 48). All of a step or
+        there they measured faster (us in a graph, hipBLASLt first, GPT-2 small's widths: fc1_fwd
+        25.2 and 24.9 with its bias and GELU still to come for hipBLASLt, qkv_fwd 25.0 and 23.7,
+        qkv_dw 29.7 and 21.0, wo_dx 15.2 and 10.3; at 64 rows 11.1 and 9.9), but for the weight
+        gradients of narrow models over long sequences, a few tiles contracting over 2048 rows or
+        more (d_model 128, 4096 rows: 33.5 and 34.3; 96, 8192: 62.6 and 68.6), where a whole step is
+        2-7 % slower (64 wide again faster: 46 and 34). Well past it the library's larger tiles win
+        (2048 rows: qkv_fwd 37 and 48; a step of 4 layers 2.67 and 2.78 ms at 1536 rows, but 2.31 and
+        2.26 at 1280, 2.18 and 2.06 at 1025, which the rule leaves to the library). All of a step or
         none, because these kernels fill a CU's LDS and gain nothing from a second stream: the whole
         step takes 6.51 ms on one stream, 6.99 on two; on hipBLASLt 6.99 and 6.74."""
         if self.library_products:
