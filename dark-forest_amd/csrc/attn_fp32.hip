@@ -169,7 +169,7 @@ __device__ __forceinline__ bool any_nonfinite(const T (&f)[N]) {
 // product, V of this one during the first. The online softmax works in the
 // log2 domain and moves its reference point only when a score exceeds it by
 // more than 8 (P stays below 2^8, the sums are fp32). Four waves a workgroup:
-// three workgroups share a CU (two above d_head 96), so that one's loads and merge
+// three workgroups share a CU (two above d_head 80), so that one's loads and merge
 // run beside another's products (eight waves measured 15-25 % slower at S = 1000).
 // Measured: H = 12, S = 1000, d_head 80 causal 29.4 us (607 us with one wave
 // per row on the vector unit); H = 8, d_head 128: S = 1024 causal 29.1 us (620
@@ -211,6 +211,14 @@ __global__ __launch_bounds__(64 * NW) void fwd_fp32_kernel(const float *__restri
 #pragma unroll
   for (int b = 0; b < DBLK; ++b) acc[b] = f32x4{};
   trim_row_frags<DBLK>(sh, lane, qf);
+  // A hidden key's score is an infinity that c2 turns into -inf, so a c2 of 0 goes
+  // into Q instead. (Masking after the scale costs the loop 2 %.)
+  if (c2 == 0.f) {
+#pragma unroll
+    for (int b = 0; b < DBLK; ++b) qf[b] *= c2;
+    c2 = 1.f;
+  }
+  const float hidden = c2 < 0.f ? INFINITY : -INFINITY;
 
   for (int t = wave; t < n_tiles; t += NW) {
     const int k0 = t * kTileKeys;
@@ -234,38 +242,37 @@ __global__ __launch_bounds__(64 * NW) void fwd_fp32_kernel(const float *__restri
     for (int z = 0; z < KS; ++z)
       load_row_frags<DBLK>(K, (t + NW) * kTileKeys + kRows * z, sh, lane, kf[z]);
 
-    // P = 2^(s c2 - m); the exact column maximum and the rescale only when a
-    // score lies more than 8 above the reference point (or none is set). Keys are
-    // hidden after the scale is applied, which may be 0 (0 * inf is NaN).
     const bool masked = k0 + kTileKeys > n_clear;
-    f32x4 x[KS];
-    auto exponents = [&](float ref) {
+    if (masked) {
 #pragma unroll
       for (int z = 0; z < KS; ++z)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x[z][r] = fmaf(s[z][r], c2, -ref);
-      if (masked) {
-#pragma unroll
-        for (int z = 0; z < KS; ++z)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (k0 + kRows * z + 4 * g + r > lim) x[z][r] = -INFINITY;
-      }
-    };
+        for (int r = 0; r < 4; ++r)
+          if (k0 + kRows * z + 4 * g + r > lim) s[z][r] = hidden;
+    }
+    // P = 2^(s c2 - m); the exact column maximum and the rescale only when a
+    // score lies more than 8 above the reference point (or none is set).
     const float m_use = m == -INFINITY ? 0.f : m;
-    exponents(m_use);
     float top = -INFINITY;
+    f32x4 x[KS];
 #pragma unroll
     for (int z = 0; z < KS; ++z)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) top = fmaxf(top, x[z][r]);
+      for (int r = 0; r < 4; ++r) {
+        x[z][r] = fmaf(s[z][r], c2, -m_use);
+        top = fmaxf(top, x[z][r]);
+      }
     if (__any(top > 8.f || m == -INFINITY)) {
       const float m_new = fmaxf(m, m_use + column_max(top));
       const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - m_new);
+      const float use = m_new == -INFINITY ? 0.f : m_new;
       l *= alpha;
 #pragma unroll
       for (int b = 0; b < DBLK; ++b) acc[b] *= alpha;
-      exponents(m_new == -INFINITY ? 0.f : m_new);
+#pragma unroll
+      for (int z = 0; z < KS; ++z)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[z][r] = fmaf(s[z][r], c2, -use);
       m = m_new;
     }
 #pragma unroll
@@ -589,11 +596,11 @@ hipError_t launch_fwd_fp32(const float *q, const float *k, const float *v, float
     constexpr int DBLK = decltype(n)::value, KS = DBLK <= 4 ? 2 : 1, NW = 4;
     const int n_blocks = (seq_len + kRows - 1) / kRows;
     const size_t grid = (size_t)n_blocks * n_heads;
-    // When every workgroup is resident at once (three per CU on 256 CUs up to
-    // d_head 96, two above) there is no later round to fill the gaps of the long ones: the short half in
-    // ascending order then lands beside them (29.1 against 34.9 us at H = 8, S =
-    // 1024, d_head 128). Larger grids run longest first (94 against 107 us at S
-    // = 2048).
+    // When every workgroup is resident at once (three per CU on 256 CUs; two above
+    // d_head 80, where the rule's last third is not) there is no later round to
+    // fill the gaps of the long ones: the short half in ascending order then lands
+    // beside them (29.1 against 34.9 us at H = 8, S = 1024, d_head 128). Larger
+    // grids run longest first (94 against 107 us at S = 2048).
     const int fold = causal && grid <= 768 ? 1 : 0;
     hipLaunchKernelGGL((fwd_fp32_kernel<DBLK, NW, KS>), linear_grid(grid), dim3(64 * NW), 0, stream, q, k, v, o, lse,
                        n_heads, seq_len, d_head, scale * kLog2e, causal ? 1 : 0, n_blocks, fold);
