@@ -20,6 +20,7 @@
 // over its lanes, gathered through LDS so that lane r holds key r for the
 // softmax, and P goes back through LDS to the V lanes. Rows that are not 4-value
 // aligned (D % 4 != 0, or an odd base) load value by value.
+// decode_few_kernel: caches of up to three keys, one wave per head.
 #include "dfattn_internal.h"
 
 #include <hip/hip_runtime.h>

@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void ln_bwd_dx_generic_kernel(const float *__r
 // per lane over its wave's `rows_per_wave` rows in order, then the four waves
 // added in order through LDS, into partial[blockIdx.x][plane][features].
 // colsum_partials_kernel adds the workgroups' partials in order. The rows are
-// read once for all of it.
+// read once for all of it. ONE: rows_per_wave is 1.
 template <int V, bool ONE>
 __global__ __launch_bounds__(256) void ln_bwd_fused_kernel(const float *__restrict__ dout, const float *__restrict__ x,
                                                            const float *__restrict__ gamma,
